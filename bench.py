@@ -490,9 +490,9 @@ def main():
         taus = workloads.source_taus(bg.t[0], bg.t[-1], args.n_tau)
     plan = gm.plan(inst_set, ks, t0, lanes=args.lanes, algo=algo, saveat=taus,
                    save=SAVE_SOURCES if taus is not None else 0)
-    chosen = {0: "wave", ALGO_WAVE: "wave", ALGO_WAVE2: "wave2", ALGO_WAVE4: "wave4", ALGO_WAVE2H: "wave2h",
+    chosen = {0: "default", ALGO_WAVE: "wave", ALGO_WAVE2: "wave2", ALGO_WAVE4: "wave4", ALGO_WAVE2H: "wave2h",
               ALGO_WAVE_ALTLU: "wave_altlu"}[plan.algo]
-    kname = {"wave": "sbz_wave_kernel", "wave2": "sbz_wave_kernel_o2", "wave4": "sbz_wave4_kernel",
+    kname = {"default": "sbz_group_save_kernel" if taus is not None else "sbz_wave_kernel", "wave": "sbz_wave_kernel", "wave2": "sbz_wave_kernel_o2", "wave4": "sbz_wave4_kernel",
              "wave2h": "sbz_wave2h_kernel", "wave_altlu": "sbz_wave_kernel_altlu"}[chosen]
     from symboltz import autotune
     if args.algo == "auto" and autotune.last_times:

@@ -86,21 +86,23 @@ typedef struct {
                                 counterpart (the reference solves one cosmology per call) */
 
 /* Kernel variants. */
-#define SBZ_ALGO_WAVE 1  /* one 64-lane wavefront per mode: chains in lanes, row-parallel border LU (default) */
+#define SBZ_ALGO_WAVE 1  /* one 64-lane wavefront per mode: chains in lanes, row-parallel border LU */
 #define SBZ_ALGO_WAVE2 3 /* SBZ_ALGO_WAVE compiled for two resident wavefronts per SIMD (throughput) */
-#define SBZ_ALGO_WAVE4 4 /* four modes per wavefront, 16 lanes each (throughput); models whose border and
-                            chains fit 16 lanes (sbz_model_capacity reports 0 otherwise), no saves */
+#define SBZ_ALGO_WAVE4 4 /* several modes per wavefront; models whose border and chains fit 16 lanes
+                            (sbz_model_capacity reports 0 otherwise), no saves.  One hierarchy per lane, 4 or 8
+                            lanes per mode, when none exceeds l = 17 and at most 4 momentum bins are
+                            massive; else four modes of 16 lanes */
 #define SBZ_ALGO_WAVE_ALTLU 5 /* SBZ_ALGO_WAVE with the other layout of the border factors in LDS: the
                                  model's default keeps strictly-lower and strictly-upper rows apart
                                  (unmasked solves) unless that costs resident workgroups, in which case
                                  it keeps one combined row per lane (masked solves, half the LDS) */
-#define SBZ_ALGO_WAVE2H 6 /* two modes per wavefront, 32 lanes each (throughput); models without the
-                             four-mode kernel whose border and chains fit 32 lanes
-                             (sbz_model_capacity reports 0 otherwise), no saves */
+#define SBZ_ALGO_WAVE2H 6 /* the same for models without SBZ_ALGO_WAVE4 whose border and chains fit 32 lanes:
+                             one hierarchy per lane, else two modes of 32 lanes */
 
 /* Solver options (solvept keywords: reltol, abstol, maxiters; src/solve.jl:543).  lanes: number of
  * resident wavefronts of the persistent grid (0: as many as fit the device).  save: SBZ_SAVE_* flags
- * (0 with saveat given: states).  algo: SBZ_ALGO_* (0: default). */
+ * (0 with saveat given: states).  algo: SBZ_ALGO_* (0: default, one hierarchy per lane for the models
+ * that have it, saves included, and SBZ_ALGO_WAVE otherwise). */
 typedef struct {
     double rtol;
     double atol;
@@ -166,8 +168,9 @@ int sbz_plan_pk(sbz_plan* p, double* pk);
 int sbz_plan_pk_modes(sbz_plan* p, const int* masks, int n_masks, int at_saves, double* out);
 int sbz_plan_destroy(sbz_plan* p);
 /* Resident capacity of a kernel variant on the model's device: modes that run at once (one per
- * wavefront for SBZ_ALGO_WAVE and SBZ_ALGO_WAVE2, four per wavefront for SBZ_ALGO_WAVE4, two for
- * SBZ_ALGO_WAVE2H), and 0 for SBZ_ALGO_WAVE4 / SBZ_ALGO_WAVE2H when the model has no such kernel.  No reference counterpart: the
+ * wavefront for SBZ_ALGO_WAVE and SBZ_ALGO_WAVE2; for SBZ_ALGO_WAVE4 and SBZ_ALGO_WAVE2H 16 or 8
+ * with one hierarchy per lane, else four and two), and 0 for SBZ_ALGO_WAVE4 / SBZ_ALGO_WAVE2H when the model
+ * has no such kernel.  No reference counterpart: the
  * autotuner (symboltz/autotune.py) uses it to decide whether higher occupancy can pay off. */
 int sbz_model_capacity(sbz_model* m, int algo, int* capacity);
 
@@ -212,11 +215,11 @@ int sbz_solve_batch_noalloc(sbz_model* m, const int* inst_set, const double* ins
 
 /* ---- mixed-model launches ---------------------------------------------------------------- */
 
-/* Several models in one persistent launch.  Replaces the per-model solve loops of a stream of
+/* Several models together.  Replaces the per-model solve loops of a stream of
  * requests over several cosmological models (solve(prob, ks) per CosmologyProblem,
- * src/solve.jl:543-569, called once per model): the solves of every model run in one launch
- * whose wavefronts pull (model, instance) entries from one queue ordered longest first across the
- * models, so the whole batch has one tail.  No reference counterpart beyond that loop.
+ * src/solve.jl:543-569, called once per model): the solves of every model run in one persistent
+ * launch, or two side by side, whose wavefronts pull (model, instance) entries from one queue ordered
+ * longest first across the models, so the whole batch has one tail.  No reference counterpart beyond that loop.
  * hip_src is the mixed-model source (symboltz.multi: each model's device code in its own namespace
  * and the kernel sbz_multi_kernel), loaded from cache_path when that file exists, else compiled
  * with hiprtc and written there; models[0..n_models) are the model handles of its families, in its
@@ -228,21 +231,21 @@ int sbz_multi_create(const char* hip_src, const char* cache_path, sbz_model* con
 /* Run plans[f] of models[f] for every family f together (one plan per model, in order; a plan may
  * hold no instances).  Plans save no states or sources (final states only) and are not tangent
  * plans.  Results land in each plan's buffers: sbz_plan_fetch and sbz_plan_pk read them as after
- * sbz_plan_run.  *kernel_ms receives the launch's duration.  With sbz_multi_attach_rows, a family
- * whose body integrates several modes per wavefront (sbz_multi_rows) and whose plan holds at least
- * twice the resident wavefronts of the attached kernel runs in that body (its wavefronts drain the
- * family's instances longest first), in a launch of the attached kernel; every other instance runs
- * in its model's one-mode body, and a run without such a family launches the one-mode kernel. */
+ * sbz_plan_run.  *kernel_ms receives the duration from the first launch to the last's end.  With
+ * sbz_multi_attach_rows, a family whose body integrates several modes per wavefront (sbz_multi_rows)
+ * runs in that body, in the attached kernel (its wavefronts drain the family's instances longest
+ * first): always with one hierarchy per lane, otherwise when its plan holds at least twice the
+ * resident wavefronts of the attached kernel.  Every other instance runs in its model's one-mode
+ * body, in the one-mode kernel beside it. */
 int sbz_multi_run(sbz_multi* mm, sbz_plan* const* plans, int n_plans, float* kernel_ms);
 /* Resident wavefronts of the one-mode mixed-model kernel (modes that run at once). */
 int sbz_multi_capacity(sbz_multi* mm, int* capacity);
 /* Attach the kernel with the several-modes bodies, sbz_multi_kernel_rows, from its own code object
  * (source and cache as sbz_multi_create; the same models in the same order).  It is a code object
- * of its own so that the one-mode kernel, which serves the latency-bound launches, keeps the
- * registers of its bodies alone.  No reference counterpart. */
+ * of its own so that each kernel's registers are its bodies' own.  No reference counterpart. */
 int sbz_multi_attach_rows(sbz_multi* mm, const char* hip_src, const char* cache_path);
-/* Modes per wavefront of each family's several-modes body: rows[f] = 4 (16-lane rows), 2 (32-lane
- * rows) or 1 (none, or no such kernel attached), f < n_models.  No reference counterpart. */
+/* Which several-modes body each family has: rows[f] = 4 (that of SBZ_ALGO_WAVE4), 2 (that of
+ * SBZ_ALGO_WAVE2H) or 1 (none, or no such kernel attached), f < n_models.  No reference counterpart. */
 int sbz_multi_rows(sbz_multi* mm, int* rows);
 int sbz_multi_destroy(sbz_multi* mm);
 

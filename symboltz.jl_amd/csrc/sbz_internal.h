@@ -26,6 +26,8 @@ struct sbz_model {
     hipFunction_t k_wave4 = nullptr;   // null when the model's border or chains exceed 16 lanes
     hipFunction_t k_wave2h = nullptr;  // two modes per wavefront; null unless the model fits 32 lanes only
     hipFunction_t k_wave_alt = nullptr;   // one mode per wavefront, the other border-factor layout
+    hipFunction_t k_group_save = nullptr; // one hierarchy per lane, with saves; null when a hierarchy is too long
+    int group_modes = 0;                  // modes per wavefront of the one-hierarchy-per-lane kernels (0: none)
     hipFunction_t k_tan = nullptr, k_pk_tan = nullptr;   // null when the tangent kernel does not fit LDS
     hipStream_t stream = nullptr;
     int device = 0;
@@ -69,14 +71,18 @@ struct SbzSolveArgsHost {
 
 // Kernel variant of tangent plans (not a caller-selectable algo: sbz_plan_create_tangent sets it).
 constexpr int SBZ_ALGO_TANGENT_INTERNAL = 100;
+// Variant of saving plans of models with one hierarchy per lane (algo 0 with saves).
+constexpr int SBZ_ALGO_GROUP_SAVE_INTERNAL = 101;
 
 // Work queues of a launch: one per XCD (instances grouped by set mod SBZ_N_XCD) when a plan has
 // several parameter sets, else one.
 constexpr int SBZ_N_XCD = 8;
 
 // Launch the persistent solve kernel of `algo` with `args` on the model's stream: grid `units`
-// wavefronts (four modes each for SBZ_ALGO_WAVE4, two for SBZ_ALGO_WAVE2H).
+// wavefronts.
 hipError_t sbz_launch_solve(sbz_model* m, int algo, SbzSolveArgsHost* args, unsigned units);
+// The variant algo 0 stands for.
+int sbz_default_algo(const sbz_model* m, bool saves);
 // Resident wavefronts of a wave variant on the model's device (the persistent grid size).
 int sbz_resident_waves(sbz_model* m, int algo);
 

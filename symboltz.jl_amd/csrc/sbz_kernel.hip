@@ -1056,7 +1056,7 @@ SBZ_DEV void sbz_wave_body(const SbzSolveArgs& a) {
     }
 }
 
-#if SBZ_WAVE4_OK || SBZ_WAVE2H_OK
+#if (SBZ_WAVE4_OK || SBZ_WAVE2H_OK) && !SBZ_GROUP_OK
 // ============================================================================================
 // Several modes per wavefront: the LN lanes of row g = lane / LN integrate one mode, for models
 // whose border and chains fit LN lanes.  LN = 16 (SBZ_ALGO_WAVE4, four modes per wavefront) or
@@ -1506,6 +1506,10 @@ SBZ_DEV void sbz_waverow_body(const SbzSolveArgs& a) {
 }
 #endif
 
+#if SBZ_GROUP_OK
+#include "sbz_group.h"
+#endif
+
 // ============================================================================================
 // Tangent solve (SBZ_ALGO_TANGENT): u and s = ∂u/∂log θ integrated together, one mode per
 // wavefront.  The augmented system  u' = J u,  s' = J s + J_θ u  is linear with the block
@@ -1911,13 +1915,27 @@ extern "C" __global__ void __launch_bounds__(64) sbz_wave_kernel_altlu(SbzSolveA
 extern "C" __global__ void __launch_bounds__(64) sbz_wave_tan_kernel(SbzSolveArgs a) { sbz_wave_tan_body(a); }
 #endif
 
+#if SBZ_GROUP_OK
+#define SBZ_ROWS_BODY(LN, a) __shared__ SbzGroupLDS S; sbz_group_run<false>(a, S)
+#else
+#define SBZ_ROWS_BODY(LN, a) sbz_waverow_body<true, LN>(a)
+#endif
 #if SBZ_WAVE4_OK
 // Four modes per wavefront, one resident wavefront per SIMD (all 512 registers per lane).
-extern "C" __global__ void __launch_bounds__(64) sbz_wave4_kernel(SbzSolveArgs a) { sbz_waverow_body<true, 16>(a); }
+extern "C" __global__ void __launch_bounds__(64) sbz_wave4_kernel(SbzSolveArgs a) { SBZ_ROWS_BODY(16, a); }
 #endif
 #if SBZ_WAVE2H_OK
 // Two modes per wavefront, for models whose border or chains exceed 16 lanes but fit 32.
-extern "C" __global__ void __launch_bounds__(64) sbz_wave2h_kernel(SbzSolveArgs a) { sbz_waverow_body<true, 32>(a); }
+extern "C" __global__ void __launch_bounds__(64) sbz_wave2h_kernel(SbzSolveArgs a) { SBZ_ROWS_BODY(32, a); }
+#endif
+#if SBZ_GROUP_OK
+// Modes per wavefront of the one-hierarchy-per-lane kernels (read by the host for the grid).
+extern "C" { __constant__ int sbz_group_modes = 64 / SBZ_GL; }
+// One hierarchy per lane, with saved states and CMB sources.
+extern "C" __global__ void __launch_bounds__(64) sbz_group_save_kernel(SbzSolveArgs a) {
+    __shared__ SbzGroupLDS S;
+    sbz_group_run<true>(a, S);
+}
 #endif
 
 // Source background table for the wave kernels: one thread per (set, save time), rows as

@@ -1,12 +1,16 @@
 // Mixed-model launches: the plans of several models (different state sizes, hierarchies and
-// species) integrated by one persistent kernel.  The code object holds every model's device code in
-// its own namespace and one kernel, sbz_multi_kernel, whose wavefronts pull entries from one queue
-// ordered by estimated cost across all models.  An entry names an instance, integrated by its
-// model's one-mode body; or, for a model with a several-modes body (two or four modes per
-// wavefront) whose plan is large enough to be throughput-bound, an entry is a ticket into that
-// body, whose rows then pull the model's instances, longest first, from the model's own queue
-// until it is empty.  Each model's plan keeps its own inputs and outputs, so
-// sbz_plan_fetch and sbz_plan_pk read the results as after sbz_plan_run.
+// species) integrated together by one persistent kernel, or by two that run side by side.  A code
+// object holds every model's device code in its own namespace and one kernel whose wavefronts pull
+// entries from one queue ordered by estimated cost across all models.  sbz_multi_kernel's entries
+// name instances, integrated by their models' one-mode bodies.  sbz_multi_kernel_rows' entries are
+// tickets into the several-modes bodies of the models that have one: the body's rows pull the
+// model's instances, longest first, from the model's own queue until it is empty.  Each model's plan
+// keeps its own inputs and outputs, so sbz_plan_fetch and sbz_plan_pk read the results as after
+// sbz_plan_run.
+//
+// Two kernels, not one with both kinds of body: in one, the compiler keeps the registers of the
+// largest body for all, and the n = 236 one-mode body spills (20 problems of five families x 64 k:
+// 346 ms in one kernel).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -31,15 +35,15 @@ struct sbz_multi {
     int device = 0;
     hipModule_t module = nullptr;        // the one-mode kernel's code object
     hipModule_t module_rows = nullptr;   // the several-modes kernel's (sbz_multi_attach_rows)
-    hipFunction_t k_multi = nullptr;   // one-mode entries only
-    hipFunction_t k_rows = nullptr;    // entries and tickets (a family with a several-modes body)
-    hipStream_t stream = nullptr;
-    hipEvent_t ev0 = nullptr, ev1 = nullptr;
+    hipFunction_t k_multi = nullptr;   // one-mode entries
+    hipFunction_t k_rows = nullptr;    // tickets (the families with a several-modes body)
+    hipStream_t stream = nullptr, stream_rows = nullptr;
+    hipEvent_t ev0 = nullptr, ev1 = nullptr, ev_rows = nullptr;
     std::vector<sbz_model*> models;
     int* d_fam = nullptr;
     int* d_inst = nullptr;
     size_t cap = 0;
-    unsigned int* d_queue = nullptr;   // [0]: the entry queue; [1 + f]: family f's own queue
+    unsigned int* d_queue = nullptr;   // [0]: instances; [1]: tickets; [2 + f]: family f's own queue
     int* d_ford = nullptr;              // the several-modes families' instance orders, longest first
     size_t ford_cap = 0;
     int rows[kMultiMaxF] = {};          // modes per wavefront of each family's body
@@ -64,7 +68,9 @@ static void multi_free(sbz_multi* mm) {
     if (mm->d_ford) (void)hipFree(mm->d_ford);
     if (mm->ev0) (void)hipEventDestroy(mm->ev0);
     if (mm->ev1) (void)hipEventDestroy(mm->ev1);
+    if (mm->ev_rows) (void)hipEventDestroy(mm->ev_rows);
     if (mm->stream) (void)hipStreamDestroy(mm->stream);
+    if (mm->stream_rows) (void)hipStreamDestroy(mm->stream_rows);
     if (mm->module) (void)hipModuleUnload(mm->module);
     if (mm->module_rows) (void)hipModuleUnload(mm->module_rows);
 }
@@ -175,7 +181,7 @@ extern "C" int sbz_multi_create(const char* hip_src, const char* cache_path, sbz
         e = hipStreamCreate(&mm->stream);
         if (e == hipSuccess) e = hipEventCreate(&mm->ev0);
         if (e == hipSuccess) e = hipEventCreate(&mm->ev1);
-        if (e == hipSuccess) e = hipMalloc((void**)&mm->d_queue, sizeof(unsigned int) * (1 + kMultiMaxF));
+        if (e == hipSuccess) e = hipMalloc((void**)&mm->d_queue, sizeof(unsigned int) * (2 + kMultiMaxF));
         if (e != hipSuccess) {
             sbz_set_error("sbz_multi_create: %s", hipGetErrorString(e));
             st = SBZ_ERR_HIP;
@@ -213,6 +219,14 @@ extern "C" int sbz_multi_attach_rows(sbz_multi* mm, const char* hip_src, const c
         }
     int resident = 0;
     st = resident_of(fn, mm->device, &resident);
+    if (st == SBZ_OK) {
+        hipError_t e = mm->stream_rows ? hipSuccess : hipStreamCreate(&mm->stream_rows);
+        if (e == hipSuccess && !mm->ev_rows) e = hipEventCreateWithFlags(&mm->ev_rows, hipEventDisableTiming);
+        if (e != hipSuccess) {
+            sbz_set_error("sbz_multi_attach_rows: %s", hipGetErrorString(e));
+            st = SBZ_ERR_HIP;
+        }
+    }
     if (st != SBZ_OK) {
         (void)hipModuleUnload(mod);
         return st;
@@ -255,12 +269,14 @@ extern "C" int sbz_multi_run(sbz_multi* mm, sbz_plan* const* plans, int n_plans,
             return SBZ_ERR_ARG;
         }
     }
-    // one queue over all plans, longest first: a mode's steps grow with k and each step's cost with
-    // the state size, so k·n orders the entries across models.  A several-modes family (rows[f] > 1)
-    // whose plan holds at least twice the resident wavefronts' worth of instances gets them sorted
-    // longest first into its own order, and one ticket per rows[f] of them, placed at the cost of
-    // the first instance the ticket's wavefront would take; below that the launch is latency-bound,
-    // where the one-mode body, fastest per mode, serves it.
+    // one queue per kernel over all its plans, longest first: a mode's steps grow with k and each
+    // step's cost with the state size, so k·n orders the entries across models.  A family that runs in its
+    // several-modes body gets its instances sorted longest first into its own order, and one ticket
+    // per `per` of them, placed at the cost of the first instance the ticket's wavefront would take.
+    // A family with one hierarchy per lane always does, with as few modes per wavefront as let all
+    // the entries be resident at once (a step takes as long for one mode as for a full wavefront);
+    // a row family (rows[f] > 1) does when its plan holds at least twice the resident wavefronts'
+    // worth of instances, and below that, where latency counts, takes the faster one-mode body.
     struct Entry {
         double cost;
         int fam, inst;
@@ -268,10 +284,24 @@ extern "C" int sbz_multi_run(sbz_multi* mm, sbz_plan* const* plans, int n_plans,
     std::vector<Entry> ent;
     std::vector<size_t> ford_off(n_plans, 0);
     std::vector<char> use_rows(n_plans, 0);
+    std::vector<int> group(n_plans, 0);
     bool rows_run = false;
     for (int f = 0; f < n_plans; ++f) {
-        use_rows[f] = mm->k_rows && mm->rows[f] > 1 && plans[f]->n_inst >= 2 * mm->resident_rows;
+        group[f] = mm->k_rows && mm->rows[f] > 1 ? plans[f]->m->group_modes : 0;
+        use_rows[f] = mm->k_rows && mm->rows[f] > 1 && plans[f]->n_inst > 0 &&
+                      (group[f] || plans[f]->n_inst >= 2 * mm->resident_rows);
         rows_run = rows_run || use_rows[f];
+    }
+    std::vector<int> per(n_plans, 1);
+    for (int share = 1; rows_run; ++share) {
+        long long entries = 0;
+        bool full = true;
+        for (int f = 0; f < n_plans; ++f) {
+            per[f] = !use_rows[f] ? 1 : group[f] ? std::min(share, group[f]) : mm->rows[f];
+            full = full && per[f] == (group[f] ? group[f] : per[f]);
+            entries += (plans[f]->n_inst + per[f] - 1) / per[f];
+        }
+        if (full || entries <= mm->resident_rows) break;
     }
     MCHK(hipSetDevice(mm->device));
     // work a plan still has on its model's stream (an sbz_plan_launch not yet waited for, a pending
@@ -294,11 +324,16 @@ extern "C" int sbz_multi_run(sbz_multi* mm, sbz_plan* const* plans, int n_plans,
         std::vector<int> ord(p->n_inst);
         for (int i = 0; i < p->n_inst; ++i) ord[i] = i;
         std::stable_sort(ord.begin(), ord.end(), [p](int x, int y) { return p->h_k[x] > p->h_k[y]; });
-        for (int j = 0; j < p->n_inst; j += mm->rows[f]) ent.push_back({p->h_k[ord[j]] * nn, f, -1});
+        for (int j = 0; j < p->n_inst; j += per[f]) ent.push_back({p->h_k[ord[j]] * nn, f, -1});
         mm->h_ford.insert(mm->h_ford.end(), ord.begin(), ord.end());
     }
-    std::stable_sort(ent.begin(), ent.end(), [](const Entry& a, const Entry& b) { return a.cost > b.cost; });
+    // instances first, then tickets, each longest first
+    std::stable_sort(ent.begin(), ent.end(), [](const Entry& a, const Entry& b) {
+        return (a.inst < 0) != (b.inst < 0) ? b.inst < 0 : a.cost > b.cost;
+    });
     const int n = (int)ent.size();
+    int n1 = 0;
+    while (n1 < n && ent[n1].inst >= 0) ++n1;
     for (int f = 0; f < n_plans; ++f) plans[f]->pk_ready = false;
     if (n == 0) {
         if (kernel_ms) *kernel_ms = 0.0f;
@@ -332,7 +367,7 @@ extern "C" int sbz_multi_run(sbz_multi* mm, sbz_plan* const* plans, int n_plans,
         MCHK(hipMemcpyAsync(mm->d_ford, mm->h_ford.data(), sizeof(int) * mm->h_ford.size(), hipMemcpyHostToDevice,
                             mm->stream));
     }
-    MCHK(hipMemsetAsync(mm->d_queue, 0, sizeof(unsigned int) * (1 + kMultiMaxF), mm->stream));
+    MCHK(hipMemsetAsync(mm->d_queue, 0, sizeof(unsigned int) * (2 + kMultiMaxF), mm->stream));
     SbzMultiArgsHost a;
     std::memset(&a, 0, sizeof(a));
     for (int f = 0; f < n_plans; ++f) {
@@ -343,20 +378,33 @@ extern "C" int sbz_multi_run(sbz_multi* mm, sbz_plan* const* plans, int n_plans,
             a.fam[f].order = nullptr;   // entries name instances directly
         } else {                        // the rows pull from the family's own queue and order
             a.fam[f].order = mm->d_ford + ford_off[f];
-            a.fam[f].queue = mm->d_queue + 1 + f;
+            a.fam[f].queue = mm->d_queue + 2 + f;
+            a.fam[f].S = (plans[f]->n_inst + per[f] - 1) / per[f];
         }
     }
     a.mfam = mm->d_fam;
     a.minst = mm->d_inst;
-    a.n = n;
+    a.n = n1;
     a.queue = mm->d_queue;
-    void* kargs[] = {&a};
-    // the kernel with the several-modes bodies only when some family runs in one: it holds more
-    // registers, which the one-mode bodies of latency-bound launches would pay for
-    const unsigned waves = (unsigned)std::max(1, std::min(n, rows_run ? mm->resident_rows : mm->resident));
+    SbzMultiArgsHost t = a;   // the tickets' table and queue
+    t.mfam = mm->d_fam + n1;
+    t.minst = mm->d_inst + n1;
+    t.n = n - n1;
+    t.queue = mm->d_queue + 1;
+    void *aargs[] = {&a}, *targs[] = {&t};
+    // the instances' kernel first: its modes take longest, the tickets' wavefronts fill the rest of
+    // the device and what the instances leave as they end
     MCHK(hipEventRecord(mm->ev0, mm->stream));
-    MCHK(hipModuleLaunchKernel(rows_run ? mm->k_rows : mm->k_multi, waves, 1, 1, 64, 1, 1, 0, mm->stream, kargs,
-                               nullptr));
+    if (n1 > 0)
+        MCHK(hipModuleLaunchKernel(mm->k_multi, (unsigned)std::min(n1, mm->resident), 1, 1, 64, 1, 1, 0, mm->stream,
+                                   aargs, nullptr));
+    if (t.n > 0) {
+        MCHK(hipStreamWaitEvent(mm->stream_rows, mm->ev0, 0));
+        MCHK(hipModuleLaunchKernel(mm->k_rows, (unsigned)std::min(t.n, mm->resident_rows), 1, 1, 64, 1, 1, 0,
+                                   mm->stream_rows, targs, nullptr));
+        MCHK(hipEventRecord(mm->ev_rows, mm->stream_rows));
+        MCHK(hipStreamWaitEvent(mm->stream, mm->ev_rows, 0));
+    }
     MCHK(hipEventRecord(mm->ev1, mm->stream));
     MCHK(hipEventSynchronize(mm->ev1));
     float ms = 0.0f;

@@ -42,9 +42,12 @@ int sbz_compile_hiprtc(const char* src, std::vector<char>& code) {
         sbz_set_error("hiprtcCreateProgram failed");
         return SBZ_ERR_COMPILE;
     }
+    // kernel_flags of symboltz/build.py
     const char* opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-                          "-packed-fp32-ops"};
-    hiprtcResult r = hiprtcCompileProgram(prog, (int)(sizeof(opts) / sizeof(opts[0])), opts);
+                          "-packed-fp32-ops", "-mllvm", "-disable-machine-licm", "-mllvm",
+                          "-sgpr-regalloc=basic"};
+    const int n_opts = (int)(sizeof(opts) / sizeof(opts[0])) - (std::strstr(src, "\n#define SBZ_GROUP_OK 1\n") ? 0 : 4);
+    hiprtcResult r = hiprtcCompileProgram(prog, n_opts, opts);
     if (r != HIPRTC_SUCCESS) {
         size_t ls = 0;
         hiprtcGetProgramLogSize(prog, &ls);
@@ -128,6 +131,16 @@ extern "C" int sbz_model_create(const char* hip_src, const sbz_model_desc* desc,
     if (hipModuleGetFunction(&m->k_wave4, m->module, "sbz_wave4_kernel") != hipSuccess) m->k_wave4 = nullptr;
     if (hipModuleGetFunction(&m->k_wave2h, m->module, "sbz_wave2h_kernel") != hipSuccess) m->k_wave2h = nullptr;
     if (hipModuleGetFunction(&m->k_wave_alt, m->module, "sbz_wave_kernel_altlu") != hipSuccess) m->k_wave_alt = nullptr;
+    {   // the one-hierarchy-per-lane kernels: with saves, and the body of the several-modes kernel
+        hipDeviceptr_t dg = nullptr;
+        size_t bytes = 0;
+        if (hipModuleGetFunction(&m->k_group_save, m->module, "sbz_group_save_kernel") != hipSuccess ||
+            hipModuleGetGlobal(&dg, &bytes, m->module, "sbz_group_modes") != hipSuccess || bytes != sizeof(int) ||
+            hipMemcpyDtoH(&m->group_modes, dg, sizeof(int)) != hipSuccess || m->group_modes < 1) {
+            m->k_group_save = nullptr;
+            m->group_modes = 0;
+        }
+    }
     if (hipModuleGetFunction(&m->k_tan, m->module, "sbz_wave_tan_kernel") != hipSuccess ||
         hipModuleGetFunction(&m->k_pk_tan, m->module, "sbz_pk_tan_kernel") != hipSuccess)
         m->k_tan = m->k_pk_tan = nullptr;
@@ -195,28 +208,46 @@ static hipError_t upload(T** dst, const T* src, size_t n) {
     return hipMemcpy(*dst, src, sizeof(T) * n, hipMemcpyHostToDevice);
 }
 
+static hipFunction_t solve_kernel(const sbz_model* m, int algo) {
+    switch (algo) {
+        case SBZ_ALGO_WAVE2: return m->k_wave2;
+        case SBZ_ALGO_WAVE4: return m->k_wave4;
+        case SBZ_ALGO_WAVE2H: return m->k_wave2h;
+        case SBZ_ALGO_WAVE_ALTLU: return m->k_wave_alt;
+        case SBZ_ALGO_GROUP_SAVE_INTERNAL: return m->k_group_save;
+        case SBZ_ALGO_TANGENT_INTERNAL: return m->k_tan;
+        default: return m->k_wave;
+    }
+}
+
+// Modes a wavefront of the variant holds at once.
+static int modes_per_wave(const sbz_model* m, int algo) {
+    const bool several = algo == SBZ_ALGO_WAVE4 || algo == SBZ_ALGO_WAVE2H || algo == SBZ_ALGO_GROUP_SAVE_INTERNAL;
+    if (!several) return 1;
+    return m->group_modes > 0 ? m->group_modes : (algo == SBZ_ALGO_WAVE4) ? 4 : 2;
+}
+
+// Variant of algo 0.  One hierarchy per lane wherever the model has it: 2 modes of n = 54 take 1.6 ms against
+// 4.9 ms in the one-mode kernel, 3000 modes 35 ms against 120 ms; n = 38: 2.3 against 3.9 and 39 against 80;
+// n = 100: 3.1 against 5.8 and (2000 modes) 60 against 129.
+int sbz_default_algo(const sbz_model* m, bool saves) {
+    if (m->group_modes == 0) return SBZ_ALGO_WAVE;
+    if (saves || (!m->k_wave4 && !m->k_wave2h)) return SBZ_ALGO_GROUP_SAVE_INTERNAL;
+    return m->k_wave4 ? SBZ_ALGO_WAVE4 : SBZ_ALGO_WAVE2H;
+}
+
 hipError_t sbz_launch_solve(sbz_model* m, int algo, SbzSolveArgsHost* args, unsigned units) {
     void* kargs[] = {args};
-    hipFunction_t kf = (algo == SBZ_ALGO_WAVE2)             ? m->k_wave2
-                       : (algo == SBZ_ALGO_WAVE4)           ? m->k_wave4
-                       : (algo == SBZ_ALGO_WAVE2H)          ? m->k_wave2h
-                       : (algo == SBZ_ALGO_WAVE_ALTLU)      ? m->k_wave_alt
-                       : (algo == SBZ_ALGO_TANGENT_INTERNAL) ? m->k_tan
-                                                            : m->k_wave;
+    hipFunction_t kf = solve_kernel(m, algo);
     return hipModuleLaunchKernel(kf, units, 1, 1, 64, 1, 1, 0, m->stream, kargs, nullptr);
 }
 
 int sbz_resident_waves(sbz_model* m, int algo) {
     int per_cu = 0, ncu = 0;
-    hipFunction_t kw = (algo == SBZ_ALGO_WAVE2)             ? m->k_wave2
-                       : (algo == SBZ_ALGO_WAVE4)           ? m->k_wave4
-                       : (algo == SBZ_ALGO_WAVE2H)          ? m->k_wave2h
-                       : (algo == SBZ_ALGO_WAVE_ALTLU)      ? m->k_wave_alt
-                       : (algo == SBZ_ALGO_TANGENT_INTERNAL) ? m->k_tan
-                                                            : m->k_wave;
+    hipFunction_t kw = solve_kernel(m, algo);
     if (!kw) return 0;
     if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kw, 64, 0) != hipSuccess || per_cu < 1)
-        per_cu = (algo == SBZ_ALGO_WAVE2) ? 8 : (algo == SBZ_ALGO_WAVE4 || algo == SBZ_ALGO_WAVE2H) ? 2 : 4;
+        per_cu = (algo == SBZ_ALGO_WAVE2) ? 8 : (m->group_modes == 0 && modes_per_wave(m, algo) > 1) ? 2 : 4;
     if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess || ncu < 1)
         ncu = 256;
     return per_cu * ncu;
@@ -230,11 +261,7 @@ extern "C" int sbz_model_capacity(sbz_model* m, int algo, int* capacity) {
         sbz_set_error("sbz_model_capacity: invalid argument");
         return SBZ_ERR_ARG;
     }
-    hipFunction_t kf = (algo == SBZ_ALGO_WAVE2)        ? m->k_wave2
-                       : (algo == SBZ_ALGO_WAVE4)      ? m->k_wave4
-                       : (algo == SBZ_ALGO_WAVE2H)     ? m->k_wave2h
-                       : (algo == SBZ_ALGO_WAVE_ALTLU) ? m->k_wave_alt
-                                                       : m->k_wave;
+    hipFunction_t kf = solve_kernel(m, algo);
     if (!kf) {
         *capacity = 0;
         return SBZ_OK;
@@ -242,7 +269,7 @@ extern "C" int sbz_model_capacity(sbz_model* m, int algo, int* capacity) {
     int per_cu = 0, ncu = 0;
     HIPCHK(hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kf, 64, 0));
     HIPCHK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, m->device));
-    *capacity = per_cu * ncu * (algo == SBZ_ALGO_WAVE4 ? 4 : algo == SBZ_ALGO_WAVE2H ? 2 : 1);
+    *capacity = per_cu * ncu * modes_per_wave(m, algo);
     return SBZ_OK;
 }
 
@@ -312,14 +339,15 @@ extern "C" int sbz_plan_create(sbz_model* m, const int* inst_set, const double* 
         delete p;
         return SBZ_ERR_ARG;
     }
-    p->algo = opts->algo ? opts->algo : SBZ_ALGO_WAVE;
+    p->algo = opts->algo ? opts->algo : sbz_default_algo(m, p->save_flags != 0);
     // `lanes`: concurrently resident wavefronts (the persistent grid)
     int lanes = opts->lanes > 0 ? opts->lanes : n_inst;
     if (opts->lanes <= 0) {
-        // persistent grid: as many wavefronts as can be resident at once, each pulling instances
-        // (four at a time for SBZ_ALGO_WAVE4, two for SBZ_ALGO_WAVE2H)
-        const int need = (p->algo == SBZ_ALGO_WAVE4) ? (n_inst + 3) / 4 : (p->algo == SBZ_ALGO_WAVE2H) ? (n_inst + 1) / 2 : n_inst;
-        lanes = std::min(need, sbz_resident_waves(m, p->algo));
+        // persistent grid: as many wavefronts as can be resident at once, each pulling instances.  The row
+        // kernels run best with every row filled; with one hierarchy per lane a step takes as long for one
+        // mode as for a full wavefront, and modes spread out end apart.
+        const int fill = m->group_modes > 0 ? 1 : modes_per_wave(m, p->algo);
+        lanes = std::min((n_inst + fill - 1) / fill, sbz_resident_waves(m, p->algo));
     }
     lanes = std::max(1, std::min(lanes, std::max(n_inst, 1)));
     p->lanes = lanes;

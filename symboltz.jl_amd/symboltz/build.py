@@ -17,6 +17,19 @@ INCLUDE = PKG.parent / "include"
 
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops"]
+# The solve kernels' step loop holds hundreds of FP64 constants (tableau, polynomials): hoisted out of
+# the loop they fill the register file and spill, materialised where they are used they cost a scalar
+# move each. Scalar registers are spilled, not split: the copy of a saved exec mask that a split leaves at the
+# head of a join block makes the vector allocator put its own copies before the mask is restored, and the
+# lanes that sat the branch out lose the copied values (tests/test_group.py looks for it in the assembly).
+# hiprtc gets the same flags in csrc/sbz_solver.cpp.
+KERNEL_FLAGS = HIP_FLAGS + ["-mllvm", "-disable-machine-licm", "-mllvm", "-sgpr-regalloc=basic"]
+
+
+def kernel_flags(src):
+    """The flags of a code object: KERNEL_FLAGS where it holds kernels with one hierarchy per lane, on whose
+    models they were checked."""
+    return KERNEL_FLAGS if "\n#define SBZ_GROUP_OK 1\n" in src else HIP_FLAGS
 
 
 def build_library(verbose=False):
@@ -40,7 +53,7 @@ def compile_code_object(src, path):
     path.parent.mkdir(exist_ok=True)
     tmp = path.with_suffix(".hip")
     tmp.write_text(src)
-    cmd = ["hipcc", "--genco"] + HIP_FLAGS + [str(tmp), "-o", str(path)]
+    cmd = ["hipcc", "--genco"] + kernel_flags(src) + [str(tmp), "-o", str(path)]
     r = subprocess.run(cmd, capture_output=True, text=True)
     tmp.unlink()
     if r.returncode != 0:

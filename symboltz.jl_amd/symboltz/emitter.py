@@ -40,6 +40,7 @@ B_NAMES = ["tau", "a", "Hc", "kd", "cs2", "rg", "rn", "rc", "rb", "rh", "ph", "I
 B_INV = ["iHc", "iIrhoP", "iIrho", "irb", "iwx1", "itau"] + [f"iE{i}" for i in range(8)]
 B_NAMES = B_NAMES + B_INV
 NB = len(B_NAMES)
+GROUP_MAX_SLOTS = 18   # longest lane of the one-hierarchy-per-lane kernel
 BIDX = {n: i for i, n in enumerate(B_NAMES)}
 
 # Per-set constants vector C[] (device: computed once per mode from the parameter vector)
@@ -1068,7 +1069,38 @@ class Emitted:
             return so
         out += tri_r("sbz_wb_tri_r", 1)
         out += tri_r("sbz_wb_tri2_r", 2)
+        out += self._emit_group()
         return out
+
+    def _emit_group(self):
+        """Layout of the one-hierarchy-per-lane kernel (csrc/sbz_group.h): the lanes' roles, hierarchy
+        ends and state components, and whether the model has that kernel."""
+        M, Lt = self.M, self.sys.L
+        lanes = [(0, M.lmax_g, 0, Lt["F"]), (1, M.lmax_g, 0, Lt["G"])]       # (kind, L, bin, first component)
+        if M.has_nu:
+            lanes.append((2, M.lmax_nu, 0, Lt["N"]))
+        if M.has_h:
+            lanes += [(3, M.lmax_h, i, Lt["H"] + i * (M.lmax_h + 1)) for i in range(M.nx)]
+        gl = 4 if len(lanes) + 1 <= 4 else 8
+        tops = sorted({ln[1] for ln in lanes})
+        other = [Lt["C"], Lt["C"] + 1, Lt["Phi"], Lt["B"], Lt["B"] + 1]
+        if M.de == "w0wa":
+            other += [Lt["X"], Lt["X"] + 1]
+        gm = max(tops[-1] + 1, len(other))
+        if gm - 1 > tops[-1]:      # the last lane has more slots than any hierarchy: a segment of empty rows
+            tops.append(gm - 1)
+        # a lane's registers hold about 12 gm + 60 doubles of the 256; five bins and more would take 16
+        # lanes, which did not come through their check on the device
+        ok = len(lanes) + 1 <= gl and gm <= GROUP_MAX_SLOTS
+        lanes = (lanes + [(5, -1, 0, -1)] * gl)[:gl - 1] + [(4, -1, 0, -1)]
+        comp = [[other[j] if kind == 4 and j < len(other) else base + j if base >= 0 and j <= L else -1
+                 for j in range(gm)] for kind, L, _, base in lanes]
+        table = lambda nm, v: f"__constant__ int {nm}[{len(v)}] = {{" + ", ".join(map(str, v)) + "};"   # noqa: E731
+        return [f"#define SBZ_GROUP_OK {1 if ok else 0}", f"#define SBZ_GL {gl}", f"#define SBZ_GM {gm}",
+                f"#define SBZ_GNTOP {len(tops)}",
+                "constexpr int sbz_gtops[SBZ_GNTOP] = {" + ", ".join(map(str, tops)) + "};",
+                table("sbz_g_kind", [ln[0] for ln in lanes]), table("sbz_g_L", [ln[1] for ln in lanes]),
+                table("sbz_g_bin", [ln[2] for ln in lanes]), table("sbz_g_comp", [q for r in comp for q in r])]
 
 
 def wave_structure(M):

@@ -5,12 +5,12 @@ namespace (the model's emitted functions spliced into the generic kernel, exactl
 own code object) and one kernel, `sbz_multi_kernel`.  Its wavefronts pull entries from a single
 queue ordered by estimated cost across the models, so a stream of requests with mixed state sizes
 is balanced over the whole device in one launch with one tail, instead of one launch (and one
-tail) per model.  An entry either names one instance, which the wavefront integrates with its
-model's one-mode Rodas5P body, or, for a model with a several-modes body (four modes per
-wavefront when its border and chains fit 16 lanes, two when they fit 32) and a plan large enough
-to be throughput-bound, is a ticket: the wavefront runs that body, whose rows pull the model's
-instances from the model's own queue (longest first) until it is empty.  Either way the results
-land in the model's plan buffers.
+tail) per model.  An entry names one instance, which the wavefront integrates with its model's
+one-mode Rodas5P body.  A second kernel beside it, `sbz_multi_kernel_rows`, takes the models with a
+several-modes body (one hierarchy per lane, or two or four modes per wavefront and a plan large
+enough to be throughput-bound): its entries are tickets, the wavefront runs that body, whose rows
+pull the model's instances from the model's own queue (longest first) until it is empty.  Either
+way the results land in the model's plan buffers.
 
 `MultiModel(gpu_models)` loads (or compiles and caches) the code object; `run(plans)` takes one
 final-state plan per model, in the same order, and runs them together.
@@ -21,7 +21,7 @@ import re
 
 from . import _lib
 from .build import INCLUDE, KCACHE
-from .solver import model_source
+from .solver import has_group, model_source
 
 MAX_FAMILIES = 8   # kMultiMaxF of csrc/sbz_multi.cpp
 
@@ -42,11 +42,12 @@ def modes_per_wave(full_src):
 
 def multi_source(models, rows_kernel=False):
     """One self-contained HIP source for the given models (see the module docstring): with the
-    one-mode kernel sbz_multi_kernel, or (rows_kernel) with sbz_multi_kernel_rows, which also takes
+    one-mode kernel sbz_multi_kernel, or (rows_kernel) with sbz_multi_kernel_rows, which takes the
     tickets.  The two are separate code objects, so each kernel's registers are its bodies' own."""
     if not 1 <= len(models) <= MAX_FAMILIES:
         raise ValueError(f"a mixed-model code object holds 1 to {MAX_FAMILIES} models")
     rows = [modes_per_wave(model_source(M).full_src) for M in models]
+    group = [has_group(model_source(M).full_src) for M in models]
     out = ["// Mixed-model code object: " + "; ".join(str(M) for M in models),
            "#ifndef __HIPCC_RTC__", "#include <hip/hip_runtime.h>", "#endif"]
     nf = len(models)
@@ -63,17 +64,18 @@ def multi_source(models, rows_kernel=False):
     lds1 = "0"
     for f in range(nf):
         lds1 = f"sbz_cmax(sizeof(sbzf{f}::WaveLDS), {lds1})"
-    lds_rows = lds1
+    lds_rows = "0"
     for f in range(nf):
         if rows[f] > 1:
-            lds_rows = f"sbz_cmax({rows[f]} * sizeof(sbzf{f}::WaveRow), {lds_rows})"
+            size = f"sizeof(sbzf{f}::SbzGroupLDS)" if group[f] else f"{rows[f]} * sizeof(sbzf{f}::WaveRow)"
+            lds_rows = f"sbz_cmax({size}, {lds_rows})"
     ns = ", ".join(f"sbzf{f}::SBZ_MULTI_N" for f in range(nf))
     rw = ", ".join(str(r) for r in rows)
     out.append(f"""
 // ---- the mixed-model kernels -----------------------------------------------------------------
 // The kernel argument: every model's solve arguments (the struct of its plan launch, identical in
-// layout in every namespace), then one queue of (model, instance) entries, longest first; the
-// instance is -1 for a ticket into a several-modes body (sbz_multi_kernel_rows only).
+// layout in every namespace), then one queue of (model, instance) entries, longest first; or, in
+// sbz_multi_kernel_rows, of tickets into the several-modes bodies (the instance is -1).
 struct SbzMultiArgs {{
     sbzf0::SbzSolveArgs fam[{MAX_FAMILIES}];
     const int* __restrict__ mfam;
@@ -89,8 +91,7 @@ __constant__ int sbz_multi_modes[{MAX_FAMILIES}] = {{{rw}}};""")
 
     def kernel(name, with_rows):
         k = [f"""
-// {"one-mode entries and tickets into the several-modes bodies" if with_rows else
-    "one-mode entries only (fewer registers: the latency-bound launches)"}
+// {"tickets into the several-modes bodies" if with_rows else "one-mode entries"}
 extern "C" __global__ void __launch_bounds__(64) {name}(SbzMultiArgs a) {{
     // the LDS of whichever model the wavefront runs: each family lays out its own rows here
     __shared__ __align__(16) unsigned char lds[{lds_rows if with_rows else lds1}];
@@ -105,20 +106,17 @@ extern "C" __global__ void __launch_bounds__(64) {name}(SbzMultiArgs a) {{
         __syncthreads();
         if (g < 0) break;
         const int f = __builtin_amdgcn_readfirstlane(a.mfam[g]);
-        const int inst = __builtin_amdgcn_readfirstlane(a.minst[g]);
-        switch (f) {{"""]
+{"" if with_rows else "        const int inst = __builtin_amdgcn_readfirstlane(a.minst[g]);" + chr(10)}        switch (f) {{"""]
         for f in range(nf):
             fa = f"reinterpret_cast<const sbzf{f}::SbzSolveArgs&>(a.fam[{f}])"
             one = (f"sbzf{f}::WaveLDS& L = *reinterpret_cast<sbzf{f}::WaveLDS*>(lds);\n"
                    f"                const sbzf{f}::WaveCtx c = sbzf{f}::sbz_wave_ctx(threadIdx.x);\n"
                    f"                sbzf{f}::sbz_wave_mode<true>({fa}, L, c, inst);")
-            if with_rows and rows[f] > 1:   # an instance, or a ticket (-1): rows drain the family's queue
-                k.append(f"""        case {f}:
-            if (inst >= 0) {{
-                {one}
-            }} else {{
-                sbzf{f}::sbz_waverow_run<true, {64 // rows[f]}>({fa}, reinterpret_cast<sbzf{f}::WaveRow*>(lds));
-            }}
+            if with_rows:
+                if rows[f] > 1:   # the body's rows drain the family's queue
+                    k.append(f"""        case {f}:
+            sbzf{f}::sbz_waverow_run<true, {64 // rows[f]}>({fa},
+                reinterpret_cast<sbzf{f}::{"SbzGroupLDS" if group[f] else "WaveRow"}*>(lds));
             break;""")
             else:
                 k.append(f"""        case {f}: {{

@@ -374,7 +374,7 @@ def solve_sets(M, par_sets, ks, bgopts=None, ptopts=None, ktini=1e-2, tauinimax=
     parameter_updater + solve, src/solve.jl:272-307 driven in a loop at test/runtests.jl:508-532).
     algo: a kernel variant (symboltz.solver.ALGO_*); None picks the autotuner when the batch holds
     at least twice the one-mode kernel's resident modes (throughput-bound: the variants differ by
-    up to 4x there), else the one-mode kernel.  Returns (P[n_sets][n_k], results, backgrounds)."""
+    up to 4x there) and the model has no kernel with one hierarchy per lane, else the library's default.  Returns (P[n_sets][n_k], results, backgrounds)."""
     ks = _check_ks(ks)
     bgopts = dict(reltol=1e-7, abstol=1e-7) | (bgopts or {})
     ptopts = dict(reltol=1e-5, abstol=1e-5, maxiters=100000) | (ptopts or {})
@@ -390,7 +390,7 @@ def solve_sets(M, par_sets, ks, bgopts=None, ptopts=None, ktini=1e-2, tauinimax=
     if algo is None:
         from .autotune import capacity
         from .solver import ALGO_AUTO, ALGO_WAVE
-        algo = ALGO_AUTO if (lanes == 0 and len(par_sets) * len(ks) >= 2 * capacity(gm, ALGO_WAVE)) else 0
+        algo = gm.group or ALGO_AUTO if (lanes == 0 and len(par_sets) * len(ks) >= 2 * capacity(gm, ALGO_WAVE)) else 0
     plan = gm.plan(np.concatenate(inst_set), np.concatenate(inst_k), np.concatenate(inst_t0),
                    rtol=ptopts["reltol"], atol=ptopts["abstol"], maxiters=ptopts["maxiters"], lanes=lanes, algo=algo)
     ms = plan.run()

@@ -123,6 +123,8 @@ def instrumented_model(M, kernel):
     from .solver import GpuModel
     em = model_source(M)
     src = wave4_source(em.full_src) if kernel == "wave4" else wave_source(em.full_src)
+    # the row body's regions, also of a model whose own kernel holds one hierarchy per lane
+    src = src.replace("#define SBZ_GROUP_OK 1", "#define SBZ_GROUP_OK 0")
     path = KCACHE / f"regions_{kernel}.hsaco"
     compile_code_object(src, path)
     saved = em.full_hash

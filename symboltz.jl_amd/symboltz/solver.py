@@ -47,7 +47,7 @@ def _deps_text():
     """The other files the emitted source is made of (their changes must change the tag)."""
     base = Path(__file__).resolve().parent.parent / "csrc"
     inc = Path(__file__).resolve().parent.parent.parent / "include"
-    return ("".join((base / f).read_text() for f in ("sbz_thermo.h", "sbz_dual.h", "sbz_rodas5p.h")) +
+    return ("".join((base / f).read_text() for f in ("sbz_thermo.h", "sbz_dual.h", "sbz_rodas5p.h", "sbz_group.h")) +
             "".join((inc / f).read_text() for f in ("sbz.h", "sbz_params.h")))
 
 
@@ -67,9 +67,9 @@ class _Opts(ctypes.Structure):
 
 ALGO_WAVE = 1
 ALGO_WAVE2 = 3
-ALGO_WAVE4 = 4   # four modes per wavefront (models whose border and chains fit 16 lanes; no saves)
+ALGO_WAVE4 = 4   # several modes per wavefront (models whose border and chains fit 16 lanes; no saves)
 ALGO_WAVE_ALTLU = 5   # ALGO_WAVE with the other layout of the border factors in LDS
-ALGO_WAVE2H = 6   # two modes per wavefront (models without ALGO_WAVE4 whose border and chains fit 32 lanes; no saves)
+ALGO_WAVE2H = 6   # several modes per wavefront (models without ALGO_WAVE4 whose border and chains fit 32 lanes; no saves)
 ALGO_AUTO = -1   # host-side: symboltz.autotune picks among the wavefront variants
 
 
@@ -99,6 +99,11 @@ def _declare(L):
     L.sbz_compile.argtypes = [ctypes.c_char_p, ctypes.c_char_p]
 
 
+def has_group(full_src):
+    """Whether a model's source has the kernels with one hierarchy per lane (SBZ_GROUP_OK)."""
+    return "\n#define SBZ_GROUP_OK 1\n" in full_src
+
+
 class GpuModel:
     def __init__(self, M):
         self.M = M
@@ -115,6 +120,12 @@ class GpuModel:
                    "sbz_model_create")
         self.h = h
         self.n_sets = 0
+        # the variant name of one hierarchy per lane for plans that save nothing (0: algo 0 only, or none)
+        self.has_group = has_group(em.full_src)
+        self.group = 0
+        for nm, algo in (("WAVE4", ALGO_WAVE4), ("WAVE2H", ALGO_WAVE2H)):
+            if self.has_group and f"\n#define SBZ_{nm}_OK 1\n" in em.full_src:
+                self.group = algo
 
     def upload_background(self, set_index, t, u, du, P):
         t = np.ascontiguousarray(t, dtype=np.float64)
@@ -126,8 +137,9 @@ class GpuModel:
         self.n_sets = max(self.n_sets, set_index + 1)
 
     def plan(self, inst_set, ks, t0, rtol=1e-5, atol=1e-5, maxiters=100000, saveat=None, lanes=0, save=0, algo=0):
-        """algo: 0 (library default, one wavefront per SIMD), ALGO_WAVE, ALGO_WAVE2, ALGO_WAVE4 or
-        ALGO_AUTO (timed choice among the variants, symboltz.autotune)."""
+        """algo: 0 (library default: one hierarchy per lane where the model has it, else ALGO_WAVE),
+        ALGO_WAVE, ALGO_WAVE2, ALGO_WAVE4, ALGO_WAVE2H or ALGO_AUTO (timed choice among the variants,
+        symboltz.autotune)."""
         if algo == ALGO_AUTO:
             from .autotune import choose
             algo = choose(self, inst_set, ks, t0, rtol, atol, maxiters, saveat, save)

@@ -77,7 +77,7 @@ def solve_spectra(X, ks_mpc=None, M=None, chunk=1024, algo=None, log=None):
             kk.append(k)
             tt.append(np.clip(np.minimum(1e-2 / k, 1e-4), bg.t[0], bg.t[-1]))
         plan = gm.plan(np.concatenate(iset), np.concatenate(kk), np.concatenate(tt),
-                       algo=ALGO_AUTO if algo is None else algo)
+                       algo=(gm.group or ALGO_AUTO) if algo is None else algo)
         if log and c0 == 0:
             from . import autotune
             log(f"kernel variant {autotune.NAMES.get(plan.algo, plan.algo)}"
