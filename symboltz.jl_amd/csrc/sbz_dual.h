@@ -57,6 +57,52 @@ SBZ_HD Dual sbz_tanh(Dual x) { double t = tanh(x.v); return Dual(t, (1.0 - t * t
 SBZ_HD Dual sbz_pow(Dual x, double p) { double y = pow(x.v, p); return Dual(y, p * y / x.v * x.d); }
 SBZ_HD Dual sbz_abs(Dual x) { return x.v < 0 ? -x : x; }
 
+// Value and N directional derivatives: the columns of a Jacobian from one evaluation.  Every derivative
+// is Dual's expression, so a column equals that of a Dual pass with the same seed.
+template <int N>
+struct DualN {
+    double v, d[N];
+    SBZ_HD DualN() : DualN(0.0) {}
+    SBZ_HD DualN(double x) : v(x) {
+        for (int j = 0; j < N; ++j) d[j] = 0.0;
+    }
+    template <class F>   // F(j): the derivative in direction j
+    static SBZ_HD DualN of(double x, F f) {
+        DualN r(x);
+        for (int j = 0; j < N; ++j) r.d[j] = f(j);
+        return r;
+    }
+};
+#define SBZ_DN template <int N> SBZ_HD DualN<N>
+#define SBZ_OF(value, deriv) DualN<N>::of(value, [&](int j) { return deriv; })
+SBZ_DN operator+(const DualN<N>& a, const DualN<N>& b) { return SBZ_OF(a.v + b.v, a.d[j] + b.d[j]); }
+SBZ_DN operator-(const DualN<N>& a, const DualN<N>& b) { return SBZ_OF(a.v - b.v, a.d[j] - b.d[j]); }
+SBZ_DN operator-(const DualN<N>& a) { return SBZ_OF(-a.v, -a.d[j]); }
+SBZ_DN operator*(const DualN<N>& a, const DualN<N>& b) { return SBZ_OF(a.v * b.v, a.d[j] * b.v + a.v * b.d[j]); }
+SBZ_DN operator/(const DualN<N>& a, const DualN<N>& b) {
+    const double r = 1.0 / b.v, q = a.v * r;
+    return SBZ_OF(q, (a.d[j] - q * b.d[j]) * r);
+}
+SBZ_DN operator+(const DualN<N>& a, double b) { return SBZ_OF(a.v + b, a.d[j]); }
+SBZ_DN operator+(double a, const DualN<N>& b) { return SBZ_OF(a + b.v, b.d[j]); }
+SBZ_DN operator-(const DualN<N>& a, double b) { return SBZ_OF(a.v - b, a.d[j]); }
+SBZ_DN operator-(double a, const DualN<N>& b) { return SBZ_OF(a - b.v, -b.d[j]); }
+SBZ_DN operator*(const DualN<N>& a, double b) { return SBZ_OF(a.v * b, a.d[j] * b); }
+SBZ_DN operator*(double a, const DualN<N>& b) { return SBZ_OF(a * b.v, a * b.d[j]); }
+SBZ_DN operator/(const DualN<N>& a, double b) { return SBZ_OF(a.v / b, a.d[j] / b); }
+SBZ_DN operator/(double a, const DualN<N>& b) {
+    const double q = a / b.v;
+    return SBZ_OF(q, -q * b.d[j] / b.v);
+}
+SBZ_DN sbz_exp(const DualN<N>& x) { const double e = exp(x.v); return SBZ_OF(e, e * x.d[j]); }
+SBZ_DN sbz_log(const DualN<N>& x) { return SBZ_OF(log(x.v), x.d[j] / x.v); }
+SBZ_DN sbz_sqrt(const DualN<N>& x) { const double s = sqrt(x.v); return SBZ_OF(s, 0.5 * x.d[j] / s); }
+SBZ_DN sbz_tanh(const DualN<N>& x) { const double t = tanh(x.v); return SBZ_OF(t, (1.0 - t * t) * x.d[j]); }
+SBZ_DN sbz_pow(const DualN<N>& x, double p) { const double y = pow(x.v, p); return SBZ_OF(y, p * y / x.v * x.d[j]); }
+SBZ_DN sbz_abs(const DualN<N>& x) { return x.v < 0 ? -x : x; }
+#undef SBZ_OF
+#undef SBZ_DN
+
 // Second-order Taylor numbers (value, d/dτ, d²/dτ²): the CMB source functions need the second
 // time derivative of the visibility function v = -κ̇ e^{-κ} (cosmologies.jl:99-105), which the
 // reference obtains by expanding D(D(...)) symbolically.
