@@ -636,14 +636,10 @@ SBZ_DEV void sbz_gsolve(const SbzGCtx& c, const SbzGFac& F, double* b) {
 // State component of a lane's slot (-1: none).
 SBZ_DEV int sbz_gcomp(const SbzGCtx& c, int l) { return sbz_g_comp[c.lane * SBZ_GM + l]; }
 
-// The groups of one wavefront integrate instances pulled from a's queue until it is empty.  With
-// SAVE, saved states and CMB sources too (the sources' background from a.srcbg).
-template <bool SAVE>
-SBZ_DEV void sbz_group_run(const SbzSolveArgs& a, SbzGroupLDS& S) {
-    constexpr int GL = SBZ_GL, NG = 64 / GL, M = SBZ_GM;
+SBZ_DEV SbzGCtx sbz_gctx() {
     SbzGCtx c;
-    c.lane = threadIdx.x & (GL - 1);
-    c.g = threadIdx.x / GL;
+    c.lane = threadIdx.x & (SBZ_GL - 1);
+    c.g = threadIdx.x / SBZ_GL;
     c.kind = sbz_g_kind[c.lane];
     c.L = sbz_g_L[c.lane];
     c.bin = sbz_g_bin[c.lane];
@@ -655,6 +651,30 @@ SBZ_DEV void sbz_group_run(const SbzSolveArgs& a, SbzGroupLDS& S) {
     c.one = c.isO ? 1.0 : 0.0;
     c.pi0 = c.isG ? 1.0 : 0.0;
     c.pi2 = (c.isF || c.isG) ? 1.0 : 0.0;
+    return c;
+}
+// the constants of wavenumber k in the set P
+SBZ_DEV void sbz_gmode(SbzGCtx& c, const double* P, double k) {
+    c.k = k;
+    c.ik = 1.0 / k;
+    c.k2 = k * k;
+    c.ik2 = 1.0 / c.k2;
+    c.x = c.isH ? P[SBZ_P_X + c.bin] : 1.0;
+    c.ix = 1.0 / c.x;
+    c.w = c.isH ? P[SBZ_P_W + c.bin] : 0.0;
+    c.dl = c.isH ? -c.x / (1.0 + exp(-c.x)) : 0.0;
+    c.al0 = (c.isF || c.isN) ? 4.0 : c.isH ? -c.dl : 3.0 * c.one;
+    c.al2 = c.one;
+    c.al3 = 3.0 * c.one;
+    c.cs2x = P[SBZ_P_CS2X];
+}
+
+// The groups of one wavefront integrate instances pulled from a's queue until it is empty.  With
+// SAVE, saved states and CMB sources too (the sources' background from a.srcbg).
+template <bool SAVE>
+SBZ_DEV void sbz_group_run(const SbzSolveArgs& a, SbzGroupLDS& S) {
+    constexpr int GL = SBZ_GL, NG = 64 / GL, M = SBZ_GM;
+    SbzGCtx c = sbz_gctx();
     double (*const gb)[SBZ_NGB] = S.f.gb[c.g];
     double (*const dgb)[SBZ_NGB] = S.f.dgb[c.g];
     double* const gc = S.f.gc[c.g];
@@ -685,21 +705,7 @@ SBZ_DEV void sbz_group_run(const SbzSolveArgs& a, SbzGroupLDS& S) {
         u[l] = 0.0;
         V.set<0>(l, 0.0);
     }
-    auto set_mode = [&](double k) SBZ_ALWAYS {
-        c.k = k;
-        c.ik = 1.0 / k;
-        c.k2 = k * k;
-        c.ik2 = 1.0 / c.k2;
-        c.x = c.isH ? P[SBZ_P_X + c.bin] : 1.0;
-        c.ix = 1.0 / c.x;
-        c.w = c.isH ? P[SBZ_P_W + c.bin] : 0.0;
-        c.dl = c.isH ? -c.x / (1.0 + exp(-c.x)) : 0.0;
-        c.al0 = (c.isF || c.isN) ? 4.0 : c.isH ? -c.dl : 3.0 * c.one;
-        c.al2 = c.one;
-        c.al3 = 3.0 * c.one;
-        c.cs2x = P[SBZ_P_CS2X];
-    };
-    set_mode(1.0);
+    sbz_gmode(c, P, 1.0);
     if (c.lane == 0) sbz_gconst(P, gc);
     auto finish = [&]() SBZ_ALWAYS {
         double* o = a.out_u + (size_t)inst * SBZ_N;
@@ -838,7 +844,7 @@ SBZ_DEV void sbz_group_run(const SbzSolveArgs& a, SbzGroupLDS& S) {
                     P = a.params + (size_t)set * SBZ_NPAR;
                     kt = a.knots + a.knot_off[set];
                     nk = a.knot_n[set];
-                    set_mode(a.inst_k[inst]);
+                    sbz_gmode(c, P, a.inst_k[inst]);
                     t1 = kt[nk - 1];
                     t = a.inst_t0[inst];
                     bidx = bidx2 = sbz_find_knot(kt, nk, t);

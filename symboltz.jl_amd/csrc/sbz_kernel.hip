@@ -1506,8 +1506,13 @@ SBZ_DEV void sbz_waverow_body(const SbzSolveArgs& a) {
 }
 #endif
 
+// The tangent solve with one hierarchy per lane: lanes of up to 12 slots, whose vectors fit 64 KB of LDS.
+#define SBZ_GTAN_OK (SBZ_GROUP_OK && SBZ_TAN_OK && SBZ_GM <= 12)
 #if SBZ_GROUP_OK
 #include "sbz_group.h"
+#endif
+#if SBZ_GTAN_OK
+#include "sbz_group_tan.h"
 #endif
 
 // ============================================================================================
@@ -1521,7 +1526,7 @@ SBZ_DEV void sbz_waverow_body(const SbzSolveArgs& a) {
 // plain solve's and s is the derivative of the discrete solution along that step sequence.
 // States only: no saves or sources.
 // ============================================================================================
-#if SBZ_TAN_OK
+#if SBZ_TAN_OK && !SBZ_GTAN_OK
 struct WaveTanLDS {
     double v[15][SBZ_N];           // primal: 0,1 U; 2,3 F; 4 DT; 5 US; 6..13 K1..K8; 14 scratch
     double w[15][SBZ_N];           // tangent, same slots
@@ -1912,7 +1917,14 @@ extern "C" __global__ void __launch_bounds__(64) sbz_wave_kernel_altlu(SbzSolveA
 
 #if SBZ_TAN_OK
 // Tangent solve, one mode and its parameter derivative per wavefront.
-extern "C" __global__ void __launch_bounds__(64) sbz_wave_tan_kernel(SbzSolveArgs a) { sbz_wave_tan_body(a); }
+extern "C" __global__ void __launch_bounds__(64) sbz_wave_tan_kernel(SbzSolveArgs a) {
+#if SBZ_GTAN_OK
+    __shared__ SbzGTanLDS S;
+    sbz_gtan_run(a, S);
+#else
+    sbz_wave_tan_body(a);
+#endif
+}
 #endif
 
 #if SBZ_GROUP_OK
