@@ -73,6 +73,9 @@ SBZ_DEV double sbz_gsum(double v) {
     return v;
 }
 
+// v of lane 0 plus v of lane 1, in these two lanes (Π_γ, which only their rows read)
+SBZ_DEV double sbz_gpair(double v) { return v + sbz_dpp<0xB1>(v); }
+
 // The background quantities the equations read at one time.
 enum {
     SBZ_GB_KD, SBZ_GB_IT, SBZ_GB_HC, SBZ_GB_IH, SBZ_GB_A2, SBZ_GB_CS, SBZ_GB_RG, SBZ_GB_RN, SBZ_GB_RC, SBZ_GB_RB,
@@ -320,8 +323,10 @@ struct SbzGCtx {
     int lane, g, kind, L, bin;             // kind 0: F, 1: G, 2: massless ν, 3: massive-ν bin, 4: fluids and Φ, 5: empty
     bool isF, isG, isN, isH, isO;
     double k, ik, ik2, k2;
-    double x, ix, w, dl;                   // momentum, weight and d ln f0/d ln x of a massive-ν bin
-    double al0, al2, al3, one;             // constant entries of α; 1 in the last lane, else 0
+    double mF, mG, mN, one;                // 1 in the lane of F, G, ν and in the last lane, else 0
+    double w0, w2;                         // a massive-ν bin's weight, and weight x² (0 elsewhere)
+    double sk0, skE, be0, beE, m1;         // s k = sk0 + skE / E; row 1's Ψ entry be0 + beE E; slip in F_1 over κ̇
+    double al0, al2, al3;                  // constant entries of α
     double pi0, pi2;                       // Π_γ = Σ pi0 u_0 + pi2 u_2
     double cs2x;
 };
@@ -338,37 +343,34 @@ struct SbzGCoef {
 
 template <class T, class LD>
 SBZ_DEV void sbz_gcoef(const SbzGCtx& c, LD ld, SbzGCoef<T>& C) {
-    const T zero(0.0);
     const T kd = ld(SBZ_GB_KD), Hc = ld(SBZ_GB_HC), A2 = ld(SBZ_GB_A2), IH = ld(SBZ_GB_IH);
     const T rg = ld(SBZ_GB_RG), cs = ld(SBZ_GB_CS);
     const T c1 = (-4.0 / 3.0 * sbzc::PI) * (A2 * IH);
     const T cq = (-8.0 * sbzc::PI * c.ik2) * A2;
-    T r0 = sbz_sel(c.isF, rg, sbz_sel(c.isN, ld(SBZ_GB_RN), sbz_sel(c.isO, ld(SBZ_GB_RC), zero)));
-    T r2 = sbz_sel(c.isO, zero, r0);
-    C.sk = T(sbz_sel(c.isF || c.isG || c.isN, c.k, 0.0));
-    C.be1 = T(sbz_sel(c.isF || c.isN, 4.0 / 3.0 * c.k, sbz_sel(c.isO, c.k2, 0.0)));
+    // what another lane holds enters with a factor 0: one instruction where a select takes two
+    T r2 = c.mF * rg + c.mN * ld(SBZ_GB_RN);
+    T r0 = r2 + c.one * ld(SBZ_GB_RC);
+    C.sk = T(c.sk0);
+    C.be1 = T(c.be0);
     if constexpr (SBZ_NX > 0) {
-        const T E = ld(SBZ_GB_E0 + c.bin), IE = ld(SBZ_GB_E0 + SBZ_NX + c.bin);
-        const T fh = ld(SBZ_GB_FH), h0 = fh * (c.w * E), h2 = fh * ((c.w * c.x * c.x) * IE);
-        const T sh = (c.k * c.x) * IE, bh = (-1.0 / 3.0 * c.k * c.ix * c.dl) * E;
-        r0 = sbz_sel(c.isH, h0, r0);
-        r2 = sbz_sel(c.isH, h2, r2);
-        C.sk = sbz_sel(c.isH, sh, C.sk);
-        C.be1 = sbz_sel(c.isH, bh, C.be1);
+        const T E = ld(SBZ_GB_E0 + c.bin), IE = ld(SBZ_GB_E0 + SBZ_NX + c.bin), fh = ld(SBZ_GB_FH);
+        r0 = r0 + fh * (c.w0 * E);
+        r2 = r2 + fh * (c.w2 * IE);
+        C.sk = C.sk + c.skE * IE;
+        C.be1 = C.be1 + c.beE * E;
     }
-    const T qh = cq * r2;
-    C.q2 = sbz_sel(c.isO, T(1.0), qh);
+    C.q2 = c.one + cq * r2;
     C.p0 = c1 * r0;
     C.p2 = -(Hc * C.q2) - (c.one * c.k2 * (1.0 / 3.0)) * IH;
     C.p3 = c.one * (c1 * ld(SBZ_GB_RB));
-    C.a01 = sbz_sel(c.isO, T(1.0), C.sk);
-    C.dd = sbz_sel(c.isF || c.isG, kd, zero);
-    C.dd0 = sbz_sel(c.isG, kd, zero);
-    C.d1 = sbz_sel(c.isO, -Hc, C.dd0);
+    C.a01 = C.sk + c.one;
+    C.dd0 = c.mG * kd;
+    C.dd = C.dd0 + c.mF * kd;
+    C.d1 = C.dd0 - c.one * Hc;
     C.top = C.dd - (c.L + 1.0) * ld(SBZ_GB_IT);
     C.ga0 = -0.5 * C.dd0;
     C.ga2 = -0.1 * C.dd;
-    C.m1 = sbz_sel(c.isF, (-4.0 / 3.0 * c.ik) * kd, zero);
+    C.m1 = c.m1 * kd;
     const T kr = c.one * (kd * (rg * ld(SBZ_GB_IRB)));
     C.m4 = (4.0 / 3.0) * kr;
     C.o33 = (-3.0 * c.one) * (Hc * cs);
@@ -382,6 +384,17 @@ SBZ_DEV void sbz_gcoef(const SbzGCtx& c, LD ld, SbzGCoef<T>& C) {
         C.x66 = -(c.one * (1.0 - 3.0 * c.cs2x)) * Hc;
         C.al5 = (3.0 * c.one) * w1;
         C.p5 = c.one * (c1 * ld(SBZ_GB_X0));
+    }
+}
+
+// The coefficients without their derivatives.
+SBZ_DEV void sbz_gvalues(const SbzGCoef<Dual>& D, SbzGCoef<double>& C) {
+    C.sk = D.sk.v; C.dd = D.dd.v; C.dd0 = D.dd0.v; C.d1 = D.d1.v; C.top = D.top.v; C.a01 = D.a01.v;
+    C.p0 = D.p0.v; C.p2 = D.p2.v; C.p3 = D.p3.v; C.q2 = D.q2.v;
+    C.be1 = D.be1.v; C.ga0 = D.ga0.v; C.ga2 = D.ga2.v; C.m1 = D.m1.v; C.m4 = D.m4.v;
+    C.o33 = D.o33.v; C.o43 = D.o43.v;
+    if constexpr (SBZ_HAS_W0WA) {
+        C.x55 = D.x55.v; C.x56 = D.x56.v; C.x65 = D.x65.v; C.x66 = D.x66.v; C.al5 = D.al5.v; C.p5 = D.p5.v;
     }
 }
 
@@ -404,7 +417,7 @@ SBZ_DEV void sbz_gsk(const SbzGCtx& c, double sk, double* skm) {
     for (int i = 1; i < SBZ_GNTOP; ++i) skm[i] = sbz_sel(c.L > sbz_gtops[i - 1], sk, 0.0);
 }
 
-// f = J u (ADD: f += J u): the rows of a lane.  Psi and Pig return Ψ and Π_γ.
+// f = J u (ADD: f += J u): the rows of a lane.  Psi and Pig return Ψ and (in the group's lanes 0 and 1) Π_γ.
 template <bool ADD>
 SBZ_DEV void sbz_grhs(const SbzGCtx& c, const SbzGCoef<double>& C, const double* u, double* f, double& Psi, double& Pig) {
     constexpr int M = SBZ_GM, GL = SBZ_GL;
@@ -416,7 +429,7 @@ SBZ_DEV void sbz_grhs(const SbzGCtx& c, const SbzGCoef<double>& C, const double*
     if constexpr (SBZ_HAS_W0WA) fp += C.p5 * u[5];
     const double dPhi = sbz_gsum<GL>(fp);
     Psi = sbz_gsum<GL>(C.q2 * u[2]);
-    Pig = sbz_gsum<GL>(c.pi0 * u[0] + c.pi2 * u[2]);
+    Pig = sbz_gpair(c.pi0 * u[0] + c.pi2 * u[2]);
     double skm[SBZ_GNTOP];
     sbz_gsk(c, C.sk, skm);
     auto row = [&](int l, double x) SBZ_ALWAYS {
@@ -458,7 +471,7 @@ SBZ_DEV void sbz_gdfdt(const SbzGCtx& c, const SbzGCoef<Dual>& C, const double* 
     }
     const double ddPhi = sbz_gsum<GL>(fp), Psi = sbz_gsum<GL>(C.q2.v * u[2]);
     dPsi = sbz_gsum<GL>(C.q2.d * u[2]);
-    const double Pig = sbz_gsum<GL>(c.pi0 * u[0] + c.pi2 * u[2]);
+    const double Pig = sbz_gpair(c.pi0 * u[0] + c.pi2 * u[2]);
     double skm[SBZ_GNTOP];
     sbz_gsk(c, C.sk.d, skm);
     out[0] = C.dd0.d * u[0] - C.a01.d * u[1] + c.al0 * ddPhi + C.ga0.d * Pig;
@@ -487,11 +500,15 @@ SBZ_DEV void sbz_gdfdt(const SbzGCtx& c, const SbzGCoef<Dual>& C, const double* 
 // Factor of u_{l-1} in row l over s k: l/(2l+1), and 1 in a hierarchy's last row.
 SBZ_DEV double sbz_gca(const SbzGCtx& c, int l) { return sbz_gtop(l) ? sbz_sel(c.L == l, 1.0, sbz_grl(l)) : sbz_grl(l); }
 
+// Lanes of up to 12 slots keep both sweeps' factors of a row, longer ones, short of registers, s k / d_l.
+constexpr bool SBZ_GKEEP = SBZ_GM <= 12;
+
 // The factored W of a lane.
 constexpr int SBZ_GNB = SBZ_HAS_W0WA ? 7 : 5;   // slots the Woodbury correction reaches
 struct SbzGFac {
     double cinv[SBZ_GM];                   // reciprocal pivots of the downward elimination
-    double cs[SBZ_GM];                     // s k / d_l (rows l >= 3)
+    double cs[SBZ_GM];                     // s k / d_l (rows l >= 3), times (l - 1's) l/(2l-1) of the downward sweep
+    double cb[SBZ_GKEEP ? SBZ_GM : 1];     // the same times l/(2l+1) (1 in the last row), of the sweep back up
     double g0, g1, h1, h2;                 // the couplings of the rows 0..2, over their pivots
     double m1, m4D, o43, i3, iD;           // F_1 ↔ θ_b, and the (δ_b, θ_b) block
     double i5, x65, x56i5, iD6;            // the (δ_X, θ_X) block
@@ -540,6 +557,7 @@ SBZ_DEV void sbz_gfactor(const SbzGCtx& c, const SbzGCoef<double>& C, double ig,
     F.m1 = C.m1;
     F.m4D = (-0.75 * c.k) * (C.m4 * F.iD);
     const double fr = sbz_gmirror<GL>(e * F.iD);
+    double cb = 0.0;
     // d_l = ig - J[l][l] + (s k)² (l+1)/(2l+1) (l+1)/(2l+3) / d_{l+1}, from the top multipole down
 #pragma unroll
     for (int l = M - 1; l >= 3; --l) {
@@ -547,11 +565,18 @@ SBZ_DEV void sbz_gfactor(const SbzGCtx& c, const SbzGCoef<double>& C, double ig,
         double cd = C.dd;
         if (sbz_gtop(l)) cd = sbz_sel(c.L == l, C.top, cd);
         double d = ig - cd;
-        if (l + 1 < M) d += (sk * sbz_grl1(l)) * (sbz_gca(c, l + 1) * F.cs[l + 1]);
+        if (l + 1 < M) d += (sk * sbz_grl1(l)) * cb;
         F.cinv[l] = sbz_rcp(d);
-        F.cs[l] = sk * F.cinv[l];
+        const double cs = sk * F.cinv[l];
+        cb = sbz_gca(c, l) * cs;
+        if constexpr (SBZ_GKEEP) {
+            F.cs[l] = sbz_grl1(l - 1) * cs;
+            F.cb[l] = cb;
+        } else {
+            F.cs[l] = cs;
+        }
     }
-    F.cinv[2] = sbz_rcp(ig - C.dd + (C.sk * (3.0 / 5.0)) * (sbz_gca(c, 3) * F.cs[3]));
+    F.cinv[2] = sbz_rcp(ig - C.dd + (C.sk * (3.0 / 5.0)) * cb);
     F.g1 = (2.0 / 3.0 * C.sk) * F.cinv[2];
     F.h2 = (2.0 / 5.0 * C.sk) * F.cinv[2];
     F.cinv[1] = sbz_rcp(ig - sbz_sel(c.isF, C.dd * fr, C.d1) + (2.0 / 3.0 * C.sk) * F.h2);
@@ -614,7 +639,7 @@ SBZ_DEV void sbz_gsolve(const SbzGCtx& c, const SbzGFac& F, double* b) {
 #pragma unroll
     for (int j = 0; j < NB; ++j) o[j] = b[j];
 #pragma unroll
-    for (int l = M - 1; l >= 3; --l) b[l - 1] -= sbz_grl1(l - 1) * (F.cs[l] * b[l]);
+    for (int l = M - 1; l >= 3; --l) b[l - 1] -= SBZ_GKEEP ? F.cs[l] * b[l] : sbz_grl1(l - 1) * (F.cs[l] * b[l]);
     o[2] = b[2];
     double y[NB];
     sbz_gborder(c, F, o, y);
@@ -628,7 +653,8 @@ SBZ_DEV void sbz_gsolve(const SbzGCtx& c, const SbzGFac& F, double* b) {
     for (int l = 0; l < 3; ++l) b[l] = y[l];
 #pragma unroll
     for (int l = 3; l < M; ++l) {
-        b[l] = b[l] * F.cinv[l] + F.cs[l] * (sbz_gca(c, l) * b[l - 1]);
+        if constexpr (SBZ_GKEEP) b[l] = b[l] * F.cinv[l] + F.cb[l] * b[l - 1];
+        else b[l] = b[l] * F.cinv[l] + F.cs[l] * (sbz_gca(c, l) * b[l - 1]);
         if (l < NB) b[l] = sbz_sel(c.isO, y[l], b[l]);
     }
 }
@@ -649,6 +675,9 @@ SBZ_DEV SbzGCtx sbz_gctx() {
     c.isH = c.kind == 3;
     c.isO = c.kind == 4;
     c.one = c.isO ? 1.0 : 0.0;
+    c.mF = c.isF ? 1.0 : 0.0;
+    c.mG = c.isG ? 1.0 : 0.0;
+    c.mN = c.isN ? 1.0 : 0.0;
     c.pi0 = c.isG ? 1.0 : 0.0;
     c.pi2 = (c.isF || c.isG) ? 1.0 : 0.0;
     return c;
@@ -659,11 +688,16 @@ SBZ_DEV void sbz_gmode(SbzGCtx& c, const double* P, double k) {
     c.ik = 1.0 / k;
     c.k2 = k * k;
     c.ik2 = 1.0 / c.k2;
-    c.x = c.isH ? P[SBZ_P_X + c.bin] : 1.0;
-    c.ix = 1.0 / c.x;
-    c.w = c.isH ? P[SBZ_P_W + c.bin] : 0.0;
-    c.dl = c.isH ? -c.x / (1.0 + exp(-c.x)) : 0.0;
-    c.al0 = (c.isF || c.isN) ? 4.0 : c.isH ? -c.dl : 3.0 * c.one;
+    const double x = c.isH ? P[SBZ_P_X + c.bin] : 0.0;      // momentum of a massive-ν bin
+    const double dl = c.isH ? -x / (1.0 + exp(-x)) : 0.0;   // d ln f0 / d ln x
+    c.w0 = c.isH ? P[SBZ_P_W + c.bin] : 0.0;
+    c.w2 = c.w0 * x * x;
+    c.sk0 = (c.isF || c.isG || c.isN) ? k : 0.0;
+    c.skE = k * x;
+    c.be0 = (c.isF || c.isN) ? 4.0 / 3.0 * k : c.isO ? c.k2 : 0.0;
+    c.beE = c.isH ? -1.0 / 3.0 * k * dl / x : 0.0;
+    c.m1 = c.isF ? -4.0 / 3.0 * c.ik : 0.0;
+    c.al0 = (c.isF || c.isN) ? 4.0 : c.isH ? -dl : 3.0 * c.one;
     c.al2 = c.one;
     c.al3 = 3.0 * c.one;
     c.cs2x = P[SBZ_P_CS2X];
@@ -989,7 +1023,7 @@ SBZ_DEV void sbz_group_run(const SbzSolveArgs& a, SbzGroupLDS& S) {
 #pragma unroll
             for (int l = 0; l < M; ++l) V.set<1>(l, DT[l]);
             SbzGCoef<double> C;
-            coef_at(0, C);
+            sbz_gvalues(D, C);
             sbz_gfactor(c, C, ig, F);
         }
         if (live) st_j++;

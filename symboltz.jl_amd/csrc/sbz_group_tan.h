@@ -318,7 +318,7 @@ SBZ_DEV void sbz_gtan_run(const SbzSolveArgs& a, SbzGTanLDS& S) {
 #pragma unroll
             for (int l = 0; l < M; ++l) K(1, l) = DT[l] + d[l];
             SbzGCoef<double> C;
-            sbz_gcoef<double>(c, [&](int i) SBZ_ALWAYS { return r0[i]; }, C);
+            sbz_gvalues(D, C);
             sbz_gfactor(c, C, ig, F);
         }
         if (live) st_j++;
