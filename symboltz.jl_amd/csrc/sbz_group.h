@@ -155,15 +155,27 @@ SBZ_DEV void sbz_gbg(const double* __restrict__ gc, const double* __restrict__ k
     const double* ku = kt + nk;
     const double* kdu = kt + 6 * (size_t)nk;
     const double tv = dval(tau);
-    // the cursor's interval and its spline data in one round trip, as sbz_pt_background
+    // the spline data of the cursor's interval and of the next in one round trip to memory: a step usually
+    // crosses a knot in some lane, and to find the interval first would take three more, one after another.
+    // Lanes of up to 12 slots only (128 x 512 massless 107 -> 101 ms): with 17 the registers are taken and
+    // the saving kernel loses more than it gains (54.0 -> 55.1 ms).
+    constexpr bool AHEAD = SBZ_GM <= 12;
+    const int i2 = !AHEAD ? idx + 1 : idx + 2 < nk ? idx + 2 : nk - 1;
     double ta = kt[idx], tb = kt[idx + 1], ua[4], ub[4], da[4], db[4];
+    const double tc = kt[i2];
+    const bool next = AHEAD && idx < nk - 2 && tv >= tb && (idx + 1 >= nk - 2 || tv < tc);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        ua[j] = ku[idx * 5 + j];
-        ub[j] = ku[(idx + 1) * 5 + j];
-        da[j] = kdu[idx * 5 + j];
-        db[j] = kdu[(idx + 1) * 5 + j];
+        const double u0 = ku[idx * 5 + j], u1 = ku[(idx + 1) * 5 + j], u2 = ku[i2 * 5 + j];
+        const double d0 = kdu[idx * 5 + j], d1 = kdu[(idx + 1) * 5 + j], d2 = kdu[i2 * 5 + j];
+        ua[j] = sbz_sel(next, u1, u0);
+        ub[j] = sbz_sel(next, u2, u1);
+        da[j] = sbz_sel(next, d1, d0);
+        db[j] = sbz_sel(next, d2, d1);
     }
+    ta = sbz_sel(next, tb, ta);
+    tb = sbz_sel(next, tc, tb);
+    idx += next;
     if ((idx > 0 && tv < ta) || (idx < nk - 2 && tv >= tb)) {
         while (idx > 0 && tv < kt[idx]) --idx;
         while (idx < nk - 2 && tv >= kt[idx + 1]) ++idx;
