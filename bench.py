@@ -387,12 +387,12 @@ def side_kernel_ms(args):
     """Kernel time of the n = 100 massive-ν workload with its sources (a few runs), reported beside
     the main workload for continuity."""
     from symboltz import workloads
-    from symboltz.solver import GpuModel, SAVE_SOURCES, ALGO_WAVE
+    from symboltz.solver import GpuModel, SAVE_SOURCES
     M, sets, ks_mpc, _ = workloads.workload("massive_nu100")
     gm = GpuModel(M)
     bgs, iset, ks, t0, _ = prepare(args, M, sets, ks_mpc, gm)
     taus = workloads.source_taus(bgs[0].t[0], bgs[0].t[-1], 2000)
-    plan = gm.plan(iset, ks, t0, saveat=taus, save=SAVE_SOURCES, algo=ALGO_WAVE)
+    plan = gm.plan(iset, ks, t0, saveat=taus, save=SAVE_SOURCES)
     plan.run()
     ms = [plan.run() for _ in range(3)]
     ok = bool(np.all(plan.fetch()["retcode"] == 0))
@@ -492,8 +492,8 @@ def main():
                    save=SAVE_SOURCES if taus is not None else 0)
     chosen = {0: "default", ALGO_WAVE: "wave", ALGO_WAVE2: "wave2", ALGO_WAVE4: "wave4", ALGO_WAVE2H: "wave2h",
               ALGO_WAVE_ALTLU: "wave_altlu"}[plan.algo]
-    kname = {"default": "sbz_group_save_kernel" if taus is not None else "sbz_wave_kernel", "wave": "sbz_wave_kernel", "wave2": "sbz_wave_kernel_o2", "wave4": "sbz_wave4_kernel",
-             "wave2h": "sbz_wave2h_kernel", "wave_altlu": "sbz_wave_kernel_altlu"}[chosen]
+    kname = {"default": "sbz_group_save_kernel", "wave": "sbz_wave_kernel", "wave2": "sbz_wave_kernel_o2",
+             "wave4": "sbz_wave4_kernel", "wave2h": "sbz_wave2h_kernel", "wave_altlu": "sbz_wave_kernel_altlu"}[chosen]
     from symboltz import autotune
     if args.algo == "auto" and autotune.last_times:
         log("autotune sample times (ms): " + ", ".join(f"{k} {v:.1f}" for k, v in autotune.last_times.items()))
@@ -547,7 +547,7 @@ def main():
     side = None
     if not args.no_side and args.workload == "lhs128":
         side_ms, side_ok = side_kernel_ms(args)
-        side = {"workload": "massive_nu100 (n=100, 1024 k, sources on 2000 tau)", "kernel": "sbz_wave_kernel",
+        side = {"workload": "massive_nu100 (n=100, 1024 k, sources on 2000 tau)", "kernel": "sbz_group_save_kernel",
                 "kernel_ms": side_ms, "all_success": side_ok, "k_mode_solves_per_s_kernel": 1024 / (side_ms * 1e-3)}
         log(f"side: massive_nu100 kernel {side_ms:.1f} ms")
         b_ms, b_ok, b_algo, b_n = side_batched_ms(args)
