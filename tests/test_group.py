@@ -143,3 +143,30 @@ def test_gpu_group_kernel_matches_one_mode_kernel(kw, n_k, lanes):
         plan.close()
     finally:
         gm.close()
+
+
+def test_emulated_group_tangent_with_two_instances_per_wavefront(massless10):
+    """Four lanes per group, so two instances share a wavefront and one slot refills: u equals the plain
+    kernel's, and s + f(τ0) dτ0/dlog θ the central difference of oracle solves at log θ ± h on the same tight
+    backgrounds (1e-3, the bar that the 8-lane model's test holds to)."""
+    from oracle import oracle
+    from symboltz import _lib
+    S = massless10
+    E = WaveEmu(model_source(S.M).full_src)
+    ks = np.array([0.5, 30.0, 4.0])
+    t0 = np.clip(np.minimum(1e-2 / ks, 1e-4), S.t[0], S.t[-1])
+    h, x, tight = 1e-3, np.log(S.pars["Omega_c0"]), []
+    for sgn in (1, -1):
+        P = models.make_params(S.M, dict(S.pars, Omega_c0=np.exp(x + sgn * h)))
+        tight.append(_lib.background_solve(P, 1e-10, 1e-10, 100000)[:4])
+    g = E.solve_tangent([(S.P, S.t, S.u, S.du)] + tight, ks, t0, 0.5 / h)
+    g1 = E.solve(S.P, S.t, S.u, S.du, ks, t0)
+    compare(dict(u=g["u"], retcode=g["retcode"], stats=g["stats"]), g1 | dict(usave=None, src=None), 3)
+    fd = []
+    for P, t, u, du in tight:
+        o = oracle.Oracle(S.M, P, t, u, du).solve(ks, t0, rtol=1e-9, atol=1e-9, maxiters=10**6)
+        assert np.all(o["retcode"] == 0)
+        fd.append(o["u"])
+    fd = (fd[0] - fd[1]) / (2 * h)
+    s = g["s"] + g["fend"] * (tight[0][1][-1] - tight[1][1][-1]) / (2 * h)
+    assert np.all(np.max(np.abs(s - fd), axis=1) < 1e-3 * np.abs(fd).max(axis=1))
