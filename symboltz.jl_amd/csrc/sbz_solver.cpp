@@ -2,7 +2,6 @@
 // ahead of time by hipcc, cached on disk), background tables, and solve plans whose inputs stay
 // resident in device memory between launches.
 #include <hip/hip_runtime.h>
-#include <hip/hiprtc.h>
 
 #include <algorithm>
 #include <cmath>
@@ -34,35 +33,6 @@ bool sbz_read_file(const char* path, std::vector<char>& out) {
     if (!f) return false;
     out.assign(std::istreambuf_iterator<char>(f), std::istreambuf_iterator<char>());
     return !out.empty();
-}
-
-int sbz_compile_hiprtc(const char* src, std::vector<char>& code) {
-    hiprtcProgram prog;
-    if (hiprtcCreateProgram(&prog, src, "sbz_model.hip", 0, nullptr, nullptr) != HIPRTC_SUCCESS) {
-        sbz_set_error("hiprtcCreateProgram failed");
-        return SBZ_ERR_COMPILE;
-    }
-    // kernel_flags of symboltz/build.py
-    const char* opts[] = {"--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-feature", "-Xclang",
-                          "-packed-fp32-ops", "-mllvm", "-disable-machine-licm", "-mllvm",
-                          "-sgpr-regalloc=basic"};
-    const int n_opts = (int)(sizeof(opts) / sizeof(opts[0])) - (std::strstr(src, "\n#define SBZ_GROUP_OK 1\n") ? 0 : 4);
-    hiprtcResult r = hiprtcCompileProgram(prog, n_opts, opts);
-    if (r != HIPRTC_SUCCESS) {
-        size_t ls = 0;
-        hiprtcGetProgramLogSize(prog, &ls);
-        std::string log(ls, '\0');
-        if (ls) hiprtcGetProgramLog(prog, &log[0]);
-        sbz_set_error("hiprtc compile failed: %.900s", log.c_str());
-        hiprtcDestroyProgram(&prog);
-        return SBZ_ERR_COMPILE;
-    }
-    size_t cs = 0;
-    hiprtcGetCodeSize(prog, &cs);
-    code.resize(cs);
-    hiprtcGetCode(prog, code.data());
-    hiprtcDestroyProgram(&prog);
-    return SBZ_OK;
 }
 
 extern "C" int sbz_compile(const char* hip_src, const char* out_path) {

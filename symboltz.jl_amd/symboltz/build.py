@@ -2,10 +2,10 @@
 
 `build_library()` compiles csrc/*.cpp into lib/libsbz_hip.so with hipcc for gfx950.
 `build_models()` emits the HIP source of the standard models and compiles each into a gfx950
-code object in _kcache/ (named by the hash of its source), so a GPU host loads them without
+code object in _kcache/ (named by the hash of its source and flags), so a GPU host loads them without
 invoking hiprtc; any other model is compiled by hiprtc on first use and cached the same way.
 """
-import os
+import hashlib
 import subprocess
 from pathlib import Path
 
@@ -22,7 +22,7 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-f
 # move each. Scalar registers are spilled, not split: the copy of a saved exec mask that a split leaves at the
 # head of a join block makes the vector allocator put its own copies before the mask is restored, and the
 # lanes that sat the branch out lose the copied values (tests/test_group.py looks for it in the assembly).
-# hiprtc gets the same flags in csrc/sbz_solver.cpp.
+# hiprtc gets the same flags in csrc/sbz_rtc.cpp.
 KERNEL_FLAGS = HIP_FLAGS + ["-mllvm", "-disable-machine-licm", "-mllvm", "-sgpr-regalloc=basic"]
 
 
@@ -32,19 +32,26 @@ def kernel_flags(src):
     return KERNEL_FLAGS if "\n#define SBZ_GROUP_OK 1\n" in src else HIP_FLAGS
 
 
+def code_hash(src):
+    """Name of a source's code object in _kcache: that of the text and of the flags it is compiled with."""
+    return hashlib.sha1((src + "\n" + " ".join(kernel_flags(src))).encode()).hexdigest()[:16]
+
+
 def build_library(verbose=False):
     LIBDIR.mkdir(exist_ok=True)
     out = LIBDIR / "libsbz_hip.so"
     srcs = [str(CSRC / f) for f in ("sbz_api.cpp", "sbz_background.cpp", "sbz_solver.cpp", "sbz_cmb.hip",
                                     "sbz_bgsolve.hip",
-                                    "sbz_mlp.hip", "sbz_noalloc.hip", "sbz_multi.cpp")]
+                                    "sbz_mlp.hip", "sbz_noalloc.hip", "sbz_multi.cpp", "sbz_rtc.cpp")]
     # -fno-math-errno: the host background solve takes square roots in line and shares equal math calls
-    cmd = ["hipcc", "-fPIC", "-shared", "-fno-math-errno", "-I", str(INCLUDE)] + HIP_FLAGS + srcs + ["-lhiprtc", "-o", str(out)]
-    r = subprocess.run(cmd, capture_output=True, text=True)
-    if r.returncode != 0:
-        raise RuntimeError(f"libsbz_hip.so build failed:\n{r.stderr[-4000:]}")
-    if verbose:
-        print("built", out)
+    cmd = ["hipcc", "-fPIC", "-shared", "-fno-math-errno", "-I", str(INCLUDE)] + HIP_FLAGS + srcs + ["-o", str(out)]
+    rtc = LIBDIR / "sbz_rtc"   # the program that the library starts to compile a source at run time
+    for cmd in (cmd, ["hipcc", "-O2", "-std=c++17", str(CSRC / "sbz_rtc_child.cpp"), "-lhiprtc", "-o", str(rtc)]):
+        r = subprocess.run(cmd, capture_output=True, text=True)
+        if r.returncode != 0:
+            raise RuntimeError(f"{Path(cmd[-1]).name} build failed:\n{r.stderr[-4000:]}")
+        if verbose:
+            print("built", cmd[-1])
     return out
 
 

@@ -30,6 +30,8 @@ from pathlib import Path
 import sympy as sp
 from sympy.printing.c import C99CodePrinter
 
+from .build import code_hash
+
 CSRC = Path(__file__).resolve().parent.parent / "csrc"
 
 # Background vector layout B[] (device: sbz_pt_background in csrc/sbz_kernel.h)
@@ -1154,5 +1156,5 @@ def kernel_source(M, fence=0):
     kern = expand_includes(CSRC / "sbz_kernel.hip")
     src = kern.replace("// @@SBZ_MODEL@@", em.src)
     em.full_src = src
-    em.full_hash = hashlib.sha1(src.encode()).hexdigest()[:16]
+    em.full_hash = code_hash(src)
     return em

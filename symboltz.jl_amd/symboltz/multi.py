@@ -16,11 +16,10 @@ way the results land in the model's plan buffers.
 final-state plan per model, in the same order, and runs them together.
 """
 import ctypes
-import hashlib
 import re
 
 from . import _lib
-from .build import INCLUDE, KCACHE
+from .build import INCLUDE, KCACHE, code_hash
 from .solver import has_group, model_source
 
 MAX_FAMILIES = 8   # kMultiMaxF of csrc/sbz_multi.cpp
@@ -135,7 +134,7 @@ extern "C" __global__ void __launch_bounds__(64) {name}(SbzMultiArgs a) {{
 
 
 def multi_cache_path(src):
-    return KCACHE / f"multi_{hashlib.sha1(src.encode()).hexdigest()[:16]}.hsaco"
+    return KCACHE / f"multi_{code_hash(src)}.hsaco"
 
 
 class MultiModel:

@@ -15,7 +15,7 @@ import numpy as np
 
 from . import _lib
 from .emitter import kernel_source
-from .build import KCACHE
+from .build import KCACHE, KERNEL_FLAGS
 
 _src_cache = {}
 
@@ -44,10 +44,11 @@ def model_source(M):
 
 
 def _deps_text():
-    """The other files the emitted source is made of (their changes must change the tag)."""
+    """What else the emitted source and its hash are made of (their changes must change the tag)."""
     base = Path(__file__).resolve().parent.parent / "csrc"
     inc = Path(__file__).resolve().parent.parent.parent / "include"
-    return ("".join((base / f).read_text() for f in ("sbz_thermo.h", "sbz_dual.h", "sbz_rodas5p.h", "sbz_group.h", "sbz_group_tan.h")) +
+    return (" ".join(KERNEL_FLAGS) +
+            "".join((base / f).read_text() for f in ("sbz_thermo.h", "sbz_dual.h", "sbz_rodas5p.h", "sbz_group.h", "sbz_group_tan.h")) +
             "".join((inc / f).read_text() for f in ("sbz.h", "sbz_params.h")))
 
 
