@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "sbz_internal.h"
+#include "sbz_multi_share.h"
 
 // Families per code object (the dimension of SbzMultiArgs::fam in the generated source).
 static constexpr int kMultiMaxF = 8;
@@ -292,17 +293,12 @@ extern "C" int sbz_multi_run(sbz_multi* mm, sbz_plan* const* plans, int n_plans,
                       (group[f] || plans[f]->n_inst >= 2 * mm->resident_rows);
         rows_run = rows_run || use_rows[f];
     }
-    std::vector<int> per(n_plans, 1);
-    for (int share = 1; rows_run; ++share) {
-        long long entries = 0;
-        bool full = true;
-        for (int f = 0; f < n_plans; ++f) {
-            per[f] = !use_rows[f] ? 1 : group[f] ? std::min(share, group[f]) : mm->rows[f];
-            full = full && per[f] == (group[f] ? group[f] : per[f]);
-            entries += (plans[f]->n_inst + per[f] - 1) / per[f];
-        }
-        if (full || entries <= mm->resident_rows) break;
+    std::vector<int> per(n_plans, 1), n_of(n_plans), rows_of(n_plans);
+    for (int f = 0; f < n_plans; ++f) {
+        n_of[f] = plans[f]->n_inst;
+        rows_of[f] = use_rows[f] ? mm->rows[f] : 1;
     }
+    if (rows_run) sbz_multi_share(n_plans, n_of.data(), rows_of.data(), group.data(), mm->resident_rows, per.data());
     MCHK(hipSetDevice(mm->device));
     // work a plan still has on its model's stream (an sbz_plan_launch not yet waited for, a pending
     // fetch) finishes before the launch writes the plan's outputs; copies of an earlier call that
