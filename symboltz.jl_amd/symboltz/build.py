@@ -101,12 +101,24 @@ def standard_models():
     ]
 
 
+def layout_models():
+    """Models whose kernels no standard model has, compiled ahead of time for their tests."""
+    from .models import LCDM
+    return [
+        LCDM(lmax=18, h=False),                           # the 16-lane row body (a hierarchy beyond l = 17)
+        LCDM(lmax=4, nx=5),                               # the 32-lane row body (more than seven hierarchies)
+        LCDM(lmax=12, h=False),                           # the one-mode tangent (lanes of more than 12 slots)
+    ]
+
+
 def standard_multis():
     """Model lists compiled ahead of time into mixed-model code objects (symboltz.multi): the mixed
-    stream's five families, and the three models of the problem-level test."""
+    stream's five families, the three models of the problem-level test, and a row family beside one with
+    one hierarchy per lane."""
     from .models import LCDM, w0waCDM
     from .workloads import mixed_families
-    return [mixed_families(), [LCDM(lmax=10, h=False), w0waCDM(lmax=6), LCDM(lmax=6)]]
+    return [mixed_families(), [LCDM(lmax=10, h=False), w0waCDM(lmax=6), LCDM(lmax=6)],
+            [LCDM(lmax=18, h=False), LCDM(lmax=10, h=False)]]
 
 
 def build_models(models=None, jobs=4, verbose=False, with_multi=None):
@@ -115,7 +127,7 @@ def build_models(models=None, jobs=4, verbose=False, with_multi=None):
     standard = models is None
     if with_multi is None:
         with_multi = standard
-    models = standard_models() if standard else models
+    models = standard_models() + layout_models() if standard else models
     KCACHE.mkdir(exist_ok=True)
     work = []
     for M in models:
