@@ -108,6 +108,8 @@ def layout_models():
         LCDM(lmax=18, h=False),                           # the 16-lane row body (a hierarchy beyond l = 17)
         LCDM(lmax=4, nx=5),                               # the 32-lane row body (more than seven hierarchies)
         LCDM(lmax=12, h=False),                           # the one-mode tangent (lanes of more than 12 slots)
+        LCDM(lmax=11),                                    # one hierarchy per lane: the longest lanes that keep both factors
+        LCDM(lmax=6, nu=False, nx=5),                     # and seven hierarchies without massless neutrinos
     ]
 
 
