@@ -20,7 +20,7 @@
 // its neighbours decides its last bit, which the step sequence follows.
 #ifdef __HIP_DEVICE_COMPILE__
 #define SBZ_BG_REUSE 0
-#else
+#elif !defined(SBZ_BG_REUSE)
 #define SBZ_BG_REUSE 1
 #endif
 
