@@ -143,13 +143,14 @@ SBZ_DEV void sbz_gconst(const double* P, double* o) {
 }
 
 // x_e of one reionization: ½ X (1 + tanh(K (f(z_re) - f(z)))) = X / (1 + exp(-2K (f(z_re) - f(z)))),
-// f(z) = (1 + z)^n (kk = -2K; the exponent is capped where the term is below 1e-300)
+// f(z) = (1 + z)^n (kk = -2K; the exponent is capped where the term is below 1e-130, nothing beside x_e, and
+// far from where the exponential times the exponent's τ-derivative, large for a narrow transition, overflows)
 template <class T>
 SBZ_DEV T sbz_greion(T opz, T sq, double xmax, double fre, double kk, double n) {
     T fz = (n == 1.5) ? sq * opz : opz;
     if (n != 1.5 && n != 1.0) fz = sbz_pow(opz, n);
     T ar = kk * (fre - fz);
-    if (dval(ar) > 690.0) ar = T(690.0);
+    if (dval(ar) > 300.0) ar = T(300.0);
     return xmax * sbz_rcp(1.0 + sbz_exp(ar));
 }
 
