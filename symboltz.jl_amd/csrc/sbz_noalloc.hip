@@ -77,8 +77,8 @@ extern "C" int sbz_solve_batch_noalloc(sbz_model* m, const int* inst_set, const 
     }
     const int algo = opts->algo ? opts->algo : sbz_default_algo(m, n_save > 0);
     if (opts->algo != 0 && algo != SBZ_ALGO_WAVE && algo != SBZ_ALGO_WAVE2) {
-        sbz_set_error("sbz_solve_batch_noalloc: only the one-mode wavefront kernels (SBZ_ALGO_WAVE, SBZ_ALGO_WAVE2) "
-                      "run without allocation");
+        sbz_set_error("sbz_solve_batch_noalloc: only algo 0 and the one-mode wavefront kernels (SBZ_ALGO_WAVE, "
+                      "SBZ_ALGO_WAVE2) run without allocation");
         return SBZ_ERR_ARG;
     }
     if (opts->save & ~SBZ_SAVE_STATES) {
