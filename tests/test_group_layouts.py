@@ -26,15 +26,15 @@ def test_emulated_layouts_match_one_mode_kernel_and_oracle(name):
     # the emulator's slot of the alternative layout runs the saving group kernel
     E = WaveEmu(src.replace("sbz_wave_kernel_altlu", "sbz_wave_kernel_other")
                 .replace("sbz_group_save_kernel", "sbz_wave_kernel_altlu"))
-    ks = np.concatenate([np.geomspace(0.05, 3.0, 4), [0.0]])
+    ks = np.concatenate([np.geomspace(0.05, 2.0, 3), [0.0]])
     t0 = np.clip(np.minimum(1e-2 / np.where(ks > 0, ks, 1.0), 1e-4), S.t[0], S.t[-1])
     saveat = np.linspace(0.05, 0.95 * S.t[-1], 5)
     w = E.solve(S.P, S.t, S.u, S.du, ks, t0, saveat=saveat, sources=True, srcbg=True)
     g = E.solve(S.P, S.t, S.u, S.du, ks, t0, saveat=saveat, sources=True, srcbg=True, altlu=True)
-    assert list(w["retcode"]) == [0] * 4 + [4]
-    compare(g, w, 4)
-    o = S.O.solve(ks[:4], t0[:4])
-    assert np.max(np.abs(g["u"][:4] - o["u"]) / np.abs(o["u"]).max(axis=1, keepdims=True)) < 1e-4
+    assert list(w["retcode"]) == [0] * 3 + [4]
+    compare(g, w, 3)
+    o = S.O.solve(ks[:3], t0[:3])
+    assert np.max(np.abs(g["u"][:3] - o["u"]) / np.abs(o["u"]).max(axis=1, keepdims=True)) < 1e-4
 
 
 @pytest.mark.gpu

@@ -33,7 +33,7 @@ def test_emulated_row_bodies_match_oracle_and_one_mode_kernel(M, variant):
     assert not has_group(src)
     E = WaveEmu(src)
     assert (E.L.emu_has_wave4(), E.L.emu_has_wave2h()) == ((1, 0) if variant == "wave4" else (0, 1))
-    ks = np.array([30.0, 0.3, 0.0, 10.0, 1.0, np.nan, 3.0] if variant == "wave4" else [10.0, 0.0, 0.3, np.nan, 3.0])
+    ks = np.array([5.0, 0.3, 0.0, 3.0, 1.0, np.nan, 2.0] if variant == "wave4" else [3.0, 0.0, 0.3, np.nan, 1.0])
     t0 = starts(S, ks)
     good = np.isfinite(ks) & (ks > 0)
     r = E.solve(S.P, S.t, S.u, S.du, ks, t0, **{variant: True})
@@ -55,7 +55,7 @@ def test_emulated_one_mode_tangent_matches_oracle_differences():
     assert "\n#define SBZ_GM 13\n" in src     # one slot more than the tangent in groups takes
     E = WaveEmu(src)
     assert E.L.emu_has_tan() == 1
-    ks = np.array([1.0, 20.0])
+    ks = np.array([1.0, 5.0])
     t0 = starts(S, ks)
     h, x, tight = 1e-3, np.log(S.pars["Omega_c0"]), []
     for sgn in (1, -1):
