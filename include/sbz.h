@@ -71,7 +71,8 @@ typedef struct sbz_plan sbz_plan;
 /* Model descriptor.  n: number of perturbation unknowns (layout: Φ, photon F_0..F_l, G_0..G_l,
  * massless ν F_0..F_l, massive ν ψ_i,0..l for each momentum bin, δ_c, θ_c, δ_b, θ_b[, δ_X, θ_X]);
  * nnz_lu: slots of the static sparse LU pattern (the algorithmic flop count's); cache_path:
- * code-object file loaded if present and written after a hiprtc compile otherwise. */
+ * code-object file loaded if present and written after a hiprtc compile otherwise (in a process of its
+ * own, by the program sbz_rtc beside the library). */
 typedef struct {
     int n;
     int nnz_lu;
@@ -90,8 +91,9 @@ typedef struct {
 #define SBZ_ALGO_WAVE2 3 /* SBZ_ALGO_WAVE compiled for two resident wavefronts per SIMD (throughput) */
 #define SBZ_ALGO_WAVE4 4 /* several modes per wavefront; models whose border and chains fit 16 lanes
                             (sbz_model_capacity reports 0 otherwise), no saves.  One hierarchy per lane, 4 or 8
-                            lanes per mode, when none exceeds l = 17 and at most 4 momentum bins are
-                            massive; else four modes of 16 lanes */
+                            lanes per mode, when none exceeds l = 17 and there are at most seven (photon
+                            temperature and polarization, massless ν, each massive momentum bin); else
+                            four modes of 16 lanes */
 #define SBZ_ALGO_WAVE_ALTLU 5 /* SBZ_ALGO_WAVE with the other layout of the border factors in LDS: the
                                  model's default keeps strictly-lower and strictly-upper rows apart
                                  (unmasked solves) unless that costs resident workgroups, in which case

@@ -13,14 +13,18 @@
 // Φ', Ψ enter as a rank-3 Woodbury correction whose functionals read slots 0..2 (0..6 in the last
 // lane), so the sweep back up over l ≥ 3 starts from the corrected values.
 //
-// The state, the stage vectors and the factors stay in registers: the step has no LDS round trip
-// but the background exchange, and no workgroup barrier inside the stages.
+// The state, the stage inputs and the factors stay in registers; f_n and as many of ∂f/∂τ, K_1..K_4 as four
+// workgroups per CU leave room for lie in LDS, one column per lane (SbzGVecs).  Lanes exchange nothing through
+// LDS but the background, and there is no workgroup barrier inside the stages.  Lanes of 17 slots (n = 100) do
+// not fit the registers: 752 B of scratch per lane, beside the moves to and from the accumulation registers.
 //
-// Bound by instruction issue: an attempt takes 5.0 k instructions at n = 54, 6.3 k at n = 38 and 8.8 k at
-// n = 100 (2.2 k of them moves to and from the accumulation registers), half of them FP64, at about six
-// cycles each, however many of the groups work; the kernels of one and of several modes before took 33 to
-// 58 us an attempt, at 39 % VALU, this one 13 to 27.  65,536 modes: n = 38 (128 sets x 512 k) 446 -> 66 ms,
-// n = 100 (64 sets x 1024 k) 2,212 -> 336 ms.  100 modes of n = 38: 77 -> 39 ms.
+// Bound by instruction issue: an attempt takes 5.1 k instructions at n = 54, 6.3 k at n = 38 and 9.1 k at
+// n = 100 (2.2 k of them moves to and from the accumulation registers), a third of them FP64 multiply-adds, at
+// five to six cycles each (eight at n = 100), however many of the groups work; the kernels of one and of several
+// modes before took 33 to 58 us an attempt, at 39 % VALU, this one 13 to 33.  65,536 modes: n = 38 (128 sets x 512 k) 446 -> 66 ms,
+// n = 100 (64 sets x 1024 k) 2,212 -> 332 ms.  100 modes of n = 38: 77 -> 39 ms.  Between those sizes, 2 and
+// 12,000 modes from 1 to 2,000 H0/c against the faster of the kernels before: n = 59 (18 slots, 4 lanes) 57 / 73 and
+// 65 / 77 ms, n = 89 (12 slots) 36 / 100 and 38 / 155 ms, n = 131 (18 slots, 8 lanes) 59 / 110 and 79 / 231 ms.
 #pragma once
 
 #ifndef SBZ_ALWAYS

@@ -11,9 +11,9 @@
 // another it would take four right-hand sides and two solves per stage.  The vectors that change
 // groups (u_in and x_u of group 0, one pass later; the groups' right-hand sides) go through LDS.
 //
-// Bound by instruction issue, as the plain step: 8.4 k instructions an attempt at n = 47, 11.5 k for two
-// instances at n = 38.  20 k for two parameters (n = 47): 277 ms a call before, 97 now, host solves of the
-// three tight backgrounds included.
+// Bound by instruction issue, as the plain step: 6.8 k instructions an attempt at n = 47 (19 us).  20 k for two
+// parameters (n = 47): 277 ms a call before, 97 now: 38 ms of kernel, the rest mostly the host's five background
+// solves (θ, and θ ± h of each parameter at a tight tolerance), one after another.
 #pragma once
 
 constexpr int SBZ_GTR = 8;                              // groups per instance

@@ -6,9 +6,11 @@
 // runs the full Rodas5P step (src/solve.jl:339 → OrdinaryDiffEqRosenbrock) on the model functions
 // emitted for this model and spliced in at the @@SBZ_MODEL@@ marker by symboltz.emitter:
 //   sbz_wave_kernel, sbz_wave_kernel_o2   one mode per 64-lane wavefront (one / two per SIMD)
-//   sbz_wave4_kernel                      four modes per wavefront, 16 lanes each
-//   sbz_wave2h_kernel                     two modes per wavefront, 32 lanes each
-//   sbz_wave_tan_kernel                   one mode and its parameter tangent per wavefront
+//   sbz_wave4_kernel, sbz_wave2h_kernel   several modes per wavefront: one hierarchy per lane (sbz_group.h, 16
+//                                         or 8 modes) where the model has it, else rows of 16 or of 32 lanes
+//   sbz_group_save_kernel                 one hierarchy per lane, with saved states and CMB sources
+//   sbz_wave_tan_kernel                   modes and their parameter tangents: in groups of lanes
+//                                         (sbz_group_tan.h) or one mode per wavefront
 // plus the source background table, P(k) and output-fill kernels.  Background spline tables (one
 // per parameter set, shared by all its modes) are read through the cache.
 #ifndef __HIPCC_RTC__  // hiprtc provides the HIP device headers itself
@@ -1059,7 +1061,7 @@ SBZ_DEV void sbz_wave_body(const SbzSolveArgs& a) {
 #if (SBZ_WAVE4_OK || SBZ_WAVE2H_OK) && !SBZ_GROUP_OK
 // ============================================================================================
 // Several modes per wavefront: the LN lanes of row g = lane / LN integrate one mode, for models
-// whose border and chains fit LN lanes.  LN = 16 (SBZ_ALGO_WAVE4, four modes per wavefront) or
+// without one hierarchy per lane whose border and chains fit LN lanes.  LN = 16 (SBZ_ALGO_WAVE4, four modes per wavefront) or
 // LN = 32 (SBZ_ALGO_WAVE2H, two modes per wavefront).  Per mode the work is sbz_wave_body's, with
 // the wavefront broadcasts and reductions in their row forms (16 lanes: DPP row_newbcast and a
 // row butterfly; 32 lanes: readlane per half and the row butterfly plus a swap of the half's two
@@ -1506,7 +1508,10 @@ SBZ_DEV void sbz_waverow_body(const SbzSolveArgs& a) {
 }
 #endif
 
-// The tangent solve with one hierarchy per lane: lanes of up to 12 slots, whose vectors fit 64 KB of LDS.
+// The tangent solve with one hierarchy per lane: lanes of up to 12 slots.  At 12, 87,656 B of LDS leave one
+// workgroup per CU and the registers spill 480 B (n = 89): 74 ms against 205 in the one-mode tangent up to 300
+// instances, 273 against 275 at 4,000; a longer lane would fall behind there.  n = 41 (massless, 12 slots):
+// 71 against 125 ms, 138 against 141 at 4,000, and behind from about 6,000 on (276 against 256 at 8,000).
 #define SBZ_GTAN_OK (SBZ_GROUP_OK && SBZ_TAN_OK && SBZ_GM <= 12)
 #if SBZ_GROUP_OK
 #include "sbz_group.h"

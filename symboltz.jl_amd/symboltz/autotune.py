@@ -9,9 +9,11 @@ For a plan it picks among the wavefront kernels:
 - SBZ_ALGO_WAVE2: one mode per wavefront, two resident per SIMD: the second hides the first's
   latency once there are more instances than SIMDs;
 - one hierarchy per lane (SBZ_ALGO_WAVE4 or SBZ_ALGO_WAVE2H of the models that have it): 4 or 8 lanes
-  per mode; faster than every other variant at any batch size, so a throughput-bound batch that
-  saves nothing takes it untimed against them.  Plans that save choose among the one-mode variants,
-  which give one another's results bit for bit; algo 0 saves with one hierarchy per lane;
+  per mode; a batch above the one-mode capacity that saves nothing takes it untimed against the others
+  (only its own 64 longest modes are run, for `last_times`).  Smaller batches and plans that save choose
+  among the one-mode variants, which give one another's results bit for bit; algo 0 takes one
+  hierarchy per lane for them too, and is two to three times faster there (100 modes of n = 38: 39
+  against 77 ms);
 - SBZ_ALGO_WAVE4: four modes per wavefront (16 lanes each), for models whose border and chains
   fit 16 lanes and plans that save nothing (models with a hierarchy beyond 17 multipoles): the per-step work that the lanes of a mode share
   (border RHS and Jacobian assembly, background) serves four modes;

