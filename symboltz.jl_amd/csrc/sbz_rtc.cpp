@@ -58,7 +58,7 @@ int sbz_compile_hiprtc(const char* src, std::vector<char>& code) {
     posix_spawn_file_actions_t fa;
     posix_spawn_file_actions_init(&fa);
     posix_spawn_file_actions_adddup2(&fa, in.fd, 0);
-    posix_spawn_file_actions_adddup2(&fa, out.fd, 1);
+    posix_spawn_file_actions_adddup2(&fa, out.fd, 3);   // after stdin's: in.fd itself may be 3
     pid_t pid = 0;
     const int e = posix_spawn(&pid, prog.c_str(), &fa, nullptr, argv.data(), environ);
     posix_spawn_file_actions_destroy(&fa);

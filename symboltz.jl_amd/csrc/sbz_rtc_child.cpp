@@ -1,6 +1,7 @@
 // sbz_rtc: compiles one HIP source with hiprtc in a process of its own (sbz_rtc.cpp starts it).
-// Source on stdin, compile options as arguments; stdout receives the code object and 'K', or the compiler's
-// log and 'E' (last, so that an output cut short has neither).
+// Source on stdin, compile options as arguments; descriptor 3 receives the code object and 'K', or the
+// compiler's log and 'E' (last, so that an output cut short has neither).  Not stdout: a library preloaded
+// into the process may print there before main.
 #include <hip/hiprtc.h>
 #include <unistd.h>
 
@@ -19,8 +20,8 @@ static bool write_all(int fd, const char* p, size_t n) {
 }
 
 int main(int argc, char** argv) {
-    const int out = dup(1);
-    dup2(2, 1);   // what the compiler prints is no part of the result
+    const int out = 3;
+    (void)dup2(2, 1);   // what the compiler prints
     // a cached result may be one of a compile whose options did not take hold
     setenv("AMD_COMGR_CACHE", "0", 1);
     std::string src, log;

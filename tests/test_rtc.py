@@ -50,6 +50,20 @@ def test_flags_are_those_of_the_ahead_of_time_build():
     assert build.code_hash(one) != build.code_hash(one.replace("\n#define SBZ_GROUP_OK 1\n", "\n#define SBZ_GROUP_OK 0\n"))
 
 
+def test_what_a_preloaded_library_prints_is_not_in_the_code(tmp_path, monkeypatch):
+    (tmp_path / "p.c").write_text("""#include <unistd.h>
+__attribute__((constructor)) static void hello(void) { if (write(1, "hello\\n", 6) < 0) _exit(9); }
+""")
+    subprocess.run(["gcc", "-shared", "-fPIC", str(tmp_path / "p.c"), "-o", str(tmp_path / "p.so")], check=True)
+    L = _lib.lib()
+    _declare(L)
+    src = b'extern "C" __global__ void k(double* p) { p[threadIdx.x] += 1.0; }'
+    assert L.sbz_compile(src, str(tmp_path / "a").encode()) == 0
+    monkeypatch.setenv("LD_PRELOAD", f"{os.environ.get('LD_PRELOAD', '')} {tmp_path / 'p.so'}".strip())
+    assert L.sbz_compile(src, str(tmp_path / "b").encode()) == 0
+    assert (tmp_path / "a").read_bytes() == (tmp_path / "b").read_bytes()
+
+
 def test_a_source_that_does_not_compile_is_an_error(tmp_path):
     L = _lib.lib()
     _declare(L)
